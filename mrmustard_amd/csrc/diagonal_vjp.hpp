@@ -250,6 +250,7 @@ __global__ __launch_bounds__(DG_THREADS) void diag_vjp_kernel(DiagVjpArgs v, int
             }
         }
         // arr0[p]'s adjoint: cotangent + diagonal pivot's g term + the off-diagonal pivots' x_2d terms
+        __syncthreads();  // the diagonal pivot's sums above still read sx of other lanes
         if (lane_ok) sx[i][slot] = gbar0;
         __syncthreads();
         if (act && i == 0) {
