@@ -82,6 +82,19 @@ int mm_hermite_batch_vjp(const double *G, const double *c, const double *dLdG, i
                          const int64_t *shape, int D, double *dA, double *db, double *dc,
                          void *workspace, size_t ws_bytes, void *stream);
 
+/* mm_hermite_batch_vjp in the convention of a gradient with respect to the
+ * conjugate (torch's): reads grad conjugated and writes conj(dA), conj(db),
+ * conj(dc).  Same workspace, same errors. */
+int mm_hermite_batch_vjp_conj(const double *G, const double *c, const double *grad, int64_t B,
+                              const int64_t *shape, int D, double *dA, double *db, double *dc,
+                              void *workspace, size_t ws_bytes, void *stream);
+
+/* out = (conj A, conj b, conj c), nA + nb + 1 complex entries in one launch
+ * (nA <= 4096, nb <= 64).  The VJPs that recompute the forward take a
+ * gradient in that convention at the conjugated triple as it is. */
+int mm_conj_triple(const double *A, int64_t nA, const double *b, int64_t nb, const double *c, double *out,
+                   void *stream);
+
 /* mm_hermite_batch_vjp without a workspace argument and without any device
  * allocation: the partial sums live in a static device buffer of
  * MM_STATIC_SCRATCH_BYTES per GPU, held until the process ends.  No

@@ -170,12 +170,14 @@ __device__ void exact_stable_forward(const Ops &t, const Lat &g, const double2 *
 }
 
 // dL/dA, dL/db, dL/dc of gradients.py:41-82, one accumulator at a time.
+// gsign = -1: the cotangent is read and the results are returned conjugated.
 template <class Ops>
 __device__ void exact_vjp(const Ops &t, const Lat &g, const double2 *G, const double2 *gg, double2 c, double2 *dA, double2 *db,
-                          double2 *dc, const double *sq) {
+                          double2 *dc, const double *sq, double gsign = 1.0) {
     const int D = g.D;
     const int64_t N = g.N;
     const double2 zero = make_double2(0.0, 0.0);
+    auto cot = [gg, gsign](int64_t p) { return make_double2(gg[p].x, gsign * gg[p].y); };
     auto wrap = [N](int64_t x) { return ((x % N) + N) % N; };
     // dLdA before the symmetrisation: entries j < i stay the zero matrix
     // entries times the cotangent
@@ -191,7 +193,7 @@ __device__ void exact_vjp(const Ops &t, const Lat &g, const double2 *G, const do
                     const double w = sq[lat_digit(g, p, i)] * sq[lat_digit(g, p, j)];
                     u = cmul(make_double2(w, 0.0), G[wrap(p - g.stride[i] - g.stride[j])]);
                 }
-                acc = cadd(acc, cmul(u, gg[p]));
+                acc = cadd(acc, cmul(u, cot(p)));
             }
             acc = t.sum(acc);
             if (t.rank == 0) dA[i * D + j] = acc;
@@ -201,24 +203,27 @@ __device__ void exact_vjp(const Ops &t, const Lat &g, const double2 *G, const do
         double2 acc = zero;
         for (int64_t p = 1 + t.rank; p < N; p += t.size) {
             const double2 u = cmul(make_double2(sq[lat_digit(g, p, i)], 0.0), G[wrap(p - g.stride[i])]);
-            acc = cadd(acc, cmul(u, gg[p]));
+            acc = cadd(acc, cmul(u, cot(p)));
         }
         acc = t.sum(acc);
         if (t.rank == 0) db[i] = acc;
     }
     double2 s = zero;
-    for (int64_t p = t.rank; p < N; p += t.size) s = cadd(s, cmul(G[p], gg[p]));
+    for (int64_t p = t.rank; p < N; p += t.size) s = cadd(s, cmul(G[p], cot(p)));
     s = t.sum(s);
     if (t.rank == 0) {
         // (dLdA + dLdA^T) / 2 with numba's complex / int division
         for (int i = 0; i < D; ++i) {
             for (int j = i; j < D; ++j) {
-                const double2 m = cdiv_promoted(cadd(dA[i * D + j], dA[j * D + i]), 2.0);
+                double2 m = cdiv_promoted(cadd(dA[i * D + j], dA[j * D + i]), 2.0);
+                m.y *= gsign;
                 dA[i * D + j] = m;
                 dA[j * D + i] = m;
             }
         }
+        for (int i = 0; i < D; ++i) db[i].y *= gsign;
         dc[0] = cdiv_py(s, c);
+        dc[0].y *= gsign;
     }
     t.sync();
 }

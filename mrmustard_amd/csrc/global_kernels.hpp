@@ -1,6 +1,6 @@
 // Kernels that work on G in global memory: the per-slab forward for lattices
-// whose slabs do not fit in LDS, the closed-form VJP reduction, and the
-// all-pivot ("stable") recurrence swept by index-sum wavefronts.
+// whose slabs do not fit in LDS, and the all-pivot ("stable") recurrence swept
+// by index-sum wavefronts.
 #pragma once
 
 #include "common.hpp"
@@ -249,12 +249,11 @@ struct Slab0Args {
     int m;
 };
 
-// Block `blk` of `nblk` (256 threads each) over the slab's points.
 template <int D>
-__device__ __forceinline__ void fwd_slab0_body(const Slab0Args &a, int64_t blk, int64_t nblk) {
+__global__ __launch_bounds__(256) void fwd_slab0_kernel(Slab0Args a) {
     const int m = a.m;
     const int64_t S = a.g.stride[0];
-    const Span sp = xcd_span(blk, nblk, S);
+    const Span sp = xcd_span(xcd_block(blockIdx.x, gridDim.x), gridDim.x, S);
     const int64_t q0 = sp.q0, inc = sp.inc, hi = sp.hi;
     if (q0 >= hi) return;
     int k[D], ki[D];
@@ -284,272 +283,9 @@ __device__ __forceinline__ void fwd_slab0_body(const Slab0Args &a, int64_t blk, 
     }
 }
 
-template <int D>
-__global__ __launch_bounds__(256) void fwd_slab0_kernel(Slab0Args a) {
-    fwd_slab0_body<D>(a, xcd_block(blockIdx.x, gridDim.x), gridDim.x);
-}
-
 __global__ void zero_c128_kernel(double2 *p, int64_t n) {
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
         p[i] = make_double2(0.0, 0.0);
-}
-
-// ------------------------------------------------------------------- the VJP
-// gradients.py:64-80 as a parallel reduction: each thread accumulates the
-// terms of its points (fused multiply-adds), a block reduces through shuffles
-// and LDS, and writes one partial per block; vjp_finalize sums the partials
-// of a triple in block order (deterministic) and symmetrises.
-struct VjpArgs {
-    Geom g;
-    const double2 *G, *gg;
-    double2 *partial;
-    const double *sq;
-    int nchunks;
-};
-
-// Accumulators of one group of pivot rows [R0, R1): dA(i, j) for R0 <= i < R1
-// and all j >= i, db_i for those rows, and dc with the first group.  Large D
-// splits the rows over several launches so each thread holds few sums.
-template <int D, int R0, int R1>
-struct RowGroup {
-    static constexpr int NT = D * (D + 1) / 2;
-    static constexpr int NA = NT + D + 1;
-    static constexpr int NROWA = (R1 - R0) * D - (R1 * (R1 - 1) - R0 * (R0 - 1)) / 2;  // sum_{i=R0}^{R1-1} (D - i)
-    static constexpr int NL = NROWA + (R1 - R0) + (R0 == 0 ? 1 : 0);
-    static __host__ __device__ constexpr int la(int i, int j) { return (i - R0) * D - (i * (i - 1) - R0 * (R0 - 1)) / 2 + (j - i); }
-    static __host__ __device__ constexpr int lb(int i) { return NROWA + (i - R0); }
-    static __host__ __device__ constexpr int lc() { return NROWA + (R1 - R0); }
-    // column of local sum l in the full layout (upper triangle of dA, db, dc)
-    static __device__ int column(int l) {
-        if (R0 == 0 && l == lc()) return NA - 1;
-        if (l >= NROWA) return NT + R0 + (l - NROWA);
-        int i = R0, off = 0;
-        while (l - off >= D - i) {
-            off += D - i;
-            ++i;
-        }
-        return i * D - i * (i - 1) / 2 + (l - off);
-    }
-};
-
-// Reduce NL sums over the block (DPP within waves, waves in order) and
-// either store or add them into the block's partial row, at the group's columns.
-template <int D, int R0, int R1, bool ADD, int NL>
-__device__ __forceinline__ void block_store_group(double2 (&acc)[NL], double2 *row) {
-    using RG = RowGroup<D, R0, R1>;
-    static_assert(NL == RG::NL, "accumulator count");
-    __shared__ double2 red[(256 / MM_WAVE) * NL];
-    wave_sum_dpp<NL>(acc);
-    const int lane = threadIdx.x & (MM_WAVE - 1), w = threadIdx.x / MM_WAVE;
-    if (lane == MM_WAVE - 1) {
-#pragma unroll
-        for (int e = 0; e < NL; ++e) red[w * NL + e] = acc[e];
-    }
-    __syncthreads();
-    if (threadIdx.x < NL) {
-        double2 t = red[threadIdx.x];
-        for (int ww = 1; ww < int(blockDim.x / MM_WAVE); ++ww) t = cadd(t, red[ww * NL + threadIdx.x]);
-        const int col = RG::column(threadIdx.x);
-        row[col] = ADD ? cadd(row[col], t) : t;
-    }
-}
-
-// gradients.py:64-80 as a parallel reduction over a whole lattice held in
-// memory.  Branch-free: a term whose digit is zero reads the point itself
-// with weight sqrt(0) = 0, so every gather of a point issues together.
-template <int D, int R0, int R1>
-__global__ __launch_bounds__(256) void vjp_kernel(VjpArgs a) {
-    using RG = RowGroup<D, R0, R1>;
-    constexpr int NL = RG::NL;
-    const int64_t t = blockIdx.y;
-    const double2 *G = a.G + t * a.g.N;
-    const double2 *gg = a.gg + t * a.g.N;
-    double2 acc[NL];
-#pragma unroll
-    for (int e = 0; e < NL; ++e) acc[e] = make_double2(0.0, 0.0);
-    const int64_t f0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const int64_t inc = int64_t(gridDim.x) * blockDim.x;
-    if (f0 < a.g.N) {
-        int64_t st[D];
-#pragma unroll
-        for (int i = 0; i < D; ++i) st[i] = a.g.stride[i];
-        int k[D], ki[D];
-        digits_of<D>(f0, a.g, 0, k);
-        digits_of<D>(inc < a.g.N ? inc : 0, a.g, 0, ki);
-        for (int64_t f = f0; f < a.g.N; f += inc) {
-            const double2 gk = gg[f];
-            if (R0 == 0) acc[RG::lc()] = cfma(G[f], gk, acc[RG::lc()]);
-#pragma unroll
-            for (int i = R0; i < R1; ++i) {
-                const int kk = k[i];
-                const double si = a.sq[kk];
-                const double2 ui = make_double2(si * gk.x, si * gk.y);
-                const int64_t p = f - (kk > 0 ? st[i] : 0);
-                acc[RG::lb(i)] = cfma(G[p], ui, acc[RG::lb(i)]);
-                const double h = 0.5 * a.sq[kk > 0 ? kk - 1 : 0];
-                const double2 t2 = G[p - (kk > 1 ? st[i] : 0)];
-                acc[RG::la(i, i)] = cfma(make_double2(h * t2.x, h * t2.y), ui, acc[RG::la(i, i)]);
-#pragma unroll
-                for (int j = i + 1; j < D; ++j) {
-                    const bool ok = kk > 0 && k[j] > 0;
-                    const double2 t3 = G[ok ? p - st[j] : f];
-                    const double w = a.sq[k[j]];
-                    acc[RG::la(i, j)] = cfma(make_double2(w * t3.x, w * t3.y), ui, acc[RG::la(i, j)]);
-                }
-            }
-            if (f + inc < a.g.N) digits_add<D>(k, ki, a.g, 0);
-        }
-    }
-    block_store_group<D, R0, R1, false>(acc, a.partial + (t * a.nchunks + blockIdx.x) * RG::NA);
-}
-
-// VJP terms of the points of level-0 slab m (k_0 = m), the three slabs given
-// as separate buffers (the recompute window); each block adds its sums into
-// its own partial row (launches are stream-ordered, so the order of the
-// additions is fixed).  Row 0 reads slabs m-1 and m-2; with m < 1 / m < 2
-// their weights are sqrt(0) = 0 and the pointers are only dereferenced at
-// valid slab-0 addresses.
-struct SlabVjpArgs {
-    Geom g;
-    const double2 *cur, *p1, *p2, *gg;
-    double2 *partial;
-    const double *sq;
-    int m;
-};
-
-// Block `blk` of `nblk` (256 threads each) adds its sums into partial row blk.
-template <int D, int R0, int R1>
-__device__ __forceinline__ void vjp_slab_body(const SlabVjpArgs &a, int64_t blk, int64_t nblk) {
-    using RG = RowGroup<D, R0, R1>;
-    constexpr int NL = RG::NL;
-    const int m = a.m;
-    const int64_t S = a.g.stride[0];
-    double2 acc[NL];
-#pragma unroll
-    for (int e = 0; e < NL; ++e) acc[e] = make_double2(0.0, 0.0);
-    const Span sp = xcd_span(blk, nblk, S);
-    const int64_t q0 = sp.q0, inc = sp.inc, hi = sp.hi;
-    if (q0 < hi) {
-        int64_t st[D];
-#pragma unroll
-        for (int i = 0; i < D; ++i) st[i] = a.g.stride[i];
-        int k[D], ki[D];
-        digits_of<D>(q0, a.g, 1, k);
-        digits_of<D>(inc < S ? inc : 0, a.g, 1, ki);
-        k[0] = m;
-        ki[0] = 0;
-        const double2 *p1 = m >= 1 ? a.p1 : a.cur;
-        const double2 *p2 = m >= 2 ? a.p2 : a.cur;
-        for (int64_t q = q0; q < hi; q += inc) {
-            const double2 gk = a.gg[q];
-            if (R0 == 0) {
-                acc[RG::lc()] = cfma(a.cur[q], gk, acc[RG::lc()]);
-                const double s0 = a.sq[m];
-                const double2 u0 = make_double2(s0 * gk.x, s0 * gk.y);
-                acc[RG::lb(0)] = cfma(p1[q], u0, acc[RG::lb(0)]);
-                const double h = 0.5 * a.sq[m > 0 ? m - 1 : 0];
-                const double2 t2 = p2[q];
-                acc[RG::la(0, 0)] = cfma(make_double2(h * t2.x, h * t2.y), u0, acc[RG::la(0, 0)]);
-#pragma unroll
-                for (int j = 1; j < D; ++j) {
-                    const double2 t3 = p1[k[j] > 0 ? q - st[j] : q];
-                    const double w = a.sq[k[j]];
-                    acc[RG::la(0, j)] = cfma(make_double2(w * t3.x, w * t3.y), u0, acc[RG::la(0, j)]);
-                }
-            }
-#pragma unroll
-            for (int i = (R0 > 1 ? R0 : 1); i < R1; ++i) {
-                const int kk = k[i];
-                const double si = a.sq[kk];
-                const double2 ui = make_double2(si * gk.x, si * gk.y);
-                const int64_t p = q - (kk > 0 ? st[i] : 0);
-                acc[RG::lb(i)] = cfma(a.cur[p], ui, acc[RG::lb(i)]);
-                const double h = 0.5 * a.sq[kk > 0 ? kk - 1 : 0];
-                const double2 t2 = a.cur[p - (kk > 1 ? st[i] : 0)];
-                acc[RG::la(i, i)] = cfma(make_double2(h * t2.x, h * t2.y), ui, acc[RG::la(i, i)]);
-#pragma unroll
-                for (int j = i + 1; j < D; ++j) {
-                    const bool ok = kk > 0 && k[j] > 0;
-                    const double2 t3 = a.cur[ok ? p - st[j] : q];
-                    const double w = a.sq[k[j]];
-                    acc[RG::la(i, j)] = cfma(make_double2(w * t3.x, w * t3.y), ui, acc[RG::la(i, j)]);
-                }
-            }
-            if (q + inc < hi) digits_add<D>(k, ki, a.g, 1);
-        }
-    }
-    block_store_group<D, R0, R1, true>(acc, a.partial + blk * RG::NA);
-}
-
-template <int D, int R0, int R1>
-__global__ __launch_bounds__(256) void vjp_slab_kernel(SlabVjpArgs a) {
-    vjp_slab_body<D, R0, R1>(a, xcd_block(blockIdx.x, gridDim.x), gridDim.x);
-}
-
-// Row groups per D: one for D <= 4, two for D = 5, 6, three for D = 7, 8.
-template <int D>
-struct RowSplit {
-    static constexpr int NG = D <= 4 ? 1 : (D <= 6 ? 2 : 3);
-    static constexpr int B1 = D <= 4 ? D : 2;
-    static constexpr int B2 = D <= 6 ? D : 4;
-};
-
-// One level-0 slab per launch, all of its work in that launch: the VJP terms
-// of slab m in every pivot-row group and (FWD) the forward of slab m + 1 from
-// slabs m and m - 1.  Logical block l (xcd_block) has role l % NR (a row
-// group, or the forward) and covers chunk l / NR of the slab, so the NR
-// blocks of one chunk run at the same time on one XCD and read the same slab
-// data: each slab is fetched about once per launch instead of once per row
-// group.  The forward writes
-// slab m + 1, which no VJP term of this launch reads.
-template <int D, bool FWD>
-__global__ __launch_bounds__(256) void slab_fused_kernel(SlabVjpArgs v, Slab0Args f) {
-    using RS = RowSplit<D>;
-    constexpr int NR = RS::NG + (FWD ? 1 : 0);
-    const int64_t l = xcd_block(blockIdx.x, gridDim.x);  // the NR roles of a chunk on one XCD
-    const int64_t role = l % NR, blk = l / NR, nblk = gridDim.x / NR;
-    if (role == 0) {
-        vjp_slab_body<D, 0, RS::B1>(v, blk, nblk);
-    } else if (RS::NG >= 2 && role == 1) {
-        if constexpr (RS::NG >= 2) vjp_slab_body<D, RS::B1, RS::B2>(v, blk, nblk);
-    } else if (RS::NG >= 3 && role == 2) {
-        if constexpr (RS::NG >= 3) vjp_slab_body<D, RS::B2, D>(v, blk, nblk);
-    } else if (FWD) {
-        fwd_slab0_body<D>(f, blk, nblk);
-    }
-}
-
-// One block per triple.  npart partial rows of NA sums each (the VJP kernel's
-// chunks, optionally followed by extra rows from other kernels).  Wave w sums
-// columns w, w + nwaves, ...: lane l adds rows l, l + 64, ... in order, then
-// the lanes combine in a fixed butterfly, so the result does not depend on
-// timing.
-template <int D>
-__global__ __launch_bounds__(1024) void vjp_finalize(const double2 *partial, int npart, const double2 *c, double2 *dA, double2 *db,
-                                                     double2 *dc) {
-    constexpr int NA = D * (D + 1) / 2 + D + 1;
-    constexpr int NT = D * (D + 1) / 2;
-    __shared__ double2 s[NA];
-    const int64_t t = blockIdx.x;
-    const double2 *p = partial + t * npart * NA;
-    const int lane = threadIdx.x & (MM_WAVE - 1);
-    const int nw = blockDim.x / MM_WAVE;
-    for (int e = threadIdx.x / MM_WAVE; e < NA; e += nw) {
-        double2 acc = make_double2(0.0, 0.0);
-#pragma unroll 8
-        for (int r = lane; r < npart; r += MM_WAVE) acc = cadd(acc, p[int64_t(r) * NA + e]);
-        acc = wave_sum(acc);
-        if (lane == 0) s[e] = acc;
-    }
-    __syncthreads();
-    if (threadIdx.x < D * D) {
-        const int i = threadIdx.x / D, j = threadIdx.x % D;
-        const int lo = i < j ? i : j, hi = i < j ? j : i;
-        const double2 m = s[lo * D - lo * (lo - 1) / 2 + (hi - lo)];
-        dA[t * D * D + threadIdx.x] = (i == j) ? m : make_double2(m.x * 0.5, m.y * 0.5);
-    }
-    if (threadIdx.x < D) db[t * D + threadIdx.x] = s[NT + threadIdx.x];
-    if (threadIdx.x == 0) dc[t] = cdiv_py(s[NA - 1], c[t]);
 }
 
 // ------------------------------------------------------------- stable sweep
@@ -802,6 +538,7 @@ struct FixArgs {
     int64_t ua, ub, uc, ug;  // per-triple strides (complex elements)
     const int *nf;           // forward: the path's flag, or NULL
     int fwd, vjp, stable;
+    double gsign;            // -1: VJP of the conjugated cotangent, results conjugated
 };
 
 __global__ __launch_bounds__(1024) void exact_fixup_kernel(FixArgs a) {
@@ -819,7 +556,7 @@ __global__ __launch_bounds__(1024) void exact_fixup_kernel(FixArgs a) {
     const double2 c = a.c[t * a.uc];
     if (a.fwd && a.stable) exact_stable_forward(ops, a.g, a.A + t * a.ua, a.b + t * a.ub, c, a.G + t * a.ug, a.sq);
     else if (a.fwd) exact_forward(ops, a.g, 0, a.A + t * a.ua, a.b + t * a.ub, c, a.G + t * a.ug, a.sq);
-    if (a.vjp) exact_vjp(ops, a.g, a.G + t * a.ug, a.gg + t * a.ug, c, a.dA + t * a.ua, a.db + t * a.ub, a.dc + t * a.uc, a.sq);
+    if (a.vjp) exact_vjp(ops, a.g, a.G + t * a.ug, a.gg + t * a.ug, c, a.dA + t * a.ua, a.db + t * a.ub, a.dc + t * a.uc, a.sq, a.gsign);
 }
 
 __global__ void zero_ints_kernel(int *p, int n) {

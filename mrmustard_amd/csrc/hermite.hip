@@ -8,6 +8,7 @@
 #include "host.hpp"
 #include "common.hpp"
 #include "global_kernels.hpp"
+#include "vjp_kernels.hpp"
 #include "jobs.hpp"
 #include "lds_kernel.hpp"
 #include "lds_launch.hpp"
@@ -493,7 +494,8 @@ Lat lat_of(const Shape &S) {
 // in the reference's arithmetic when the path met a non-finite value (the
 // forward's flag nf, or a non-finite dc when the VJP was computed).
 int launch_fixup(const Shape &S, int64_t B, const double *A, const double *b, const double *c, const double *g, double *G, double *dA,
-                 double *db, double *dc, const int *nf, bool fwd, bool vjp, const DevState *ds, hipStream_t s, bool stable = false) {
+                 double *db, double *dc, const int *nf, bool fwd, bool vjp, const DevState *ds, hipStream_t s, bool stable = false,
+                 bool conj = false) {
     if (B < 1) return MM_OK;
     if (B > 0x7fffffff) return fail(MM_ERR_UNSUPPORTED, "too many triples for one launch");
     FixArgs a;
@@ -516,6 +518,7 @@ int launch_fixup(const Shape &S, int64_t B, const double *A, const double *b, co
     a.fwd = fwd;
     a.vjp = vjp;
     a.stable = stable;
+    a.gsign = conj ? -1.0 : 1.0;
     hipLaunchKernelGGL(exact_fixup_kernel, dim3(unsigned(B)), dim3(1024), 0, s, a);
     LAUNCH_CHECK("exact_fixup_kernel");
     return MM_OK;
@@ -523,138 +526,147 @@ int launch_fixup(const Shape &S, int64_t B, const double *A, const double *b, co
 
 // ------------------------------------------------------------------ VJP path
 
-// One launch per pivot-row group (RowSplit) of the VJP kernels.
-template <int D>
-void launch_vjp_groups(const VjpArgs &a, dim3 grid, hipStream_t s) {
-    using RS = RowSplit<D>;
-    hipLaunchKernelGGL((vjp_kernel<D, 0, RS::B1>), grid, dim3(256), 0, s, a);
-    if constexpr (RS::NG >= 2) hipLaunchKernelGGL((vjp_kernel<D, RS::B1, RS::B2>), grid, dim3(256), 0, s, a);
-    if constexpr (RS::NG >= 3) hipLaunchKernelGGL((vjp_kernel<D, RS::B2, D>), grid, dim3(256), 0, s, a);
-}
-
 // Threads of the finalize block of each triple: one wave per sum column for
 // few triples, four waves when many triples fill the GPU anyway.
 int finalize_threads(int64_t B) { return B >= 64 ? 256 : 1024; }
 
-int vjp_chunks(int64_t N, int64_t B) {
+// Largest workspace that a VJP of this size was ever asked for: callers with
+// buffers of this size, and the static buffer's limit, keep it as their measure.
+int vjp_chunks_min_ws(int64_t N, int64_t B) {
     int64_t per = 256 * 8;
     int64_t want = (N + per - 1) / per;
     int64_t cap = std::max<int64_t>(1, 8192 / std::max<int64_t>(B, 1));
     return int(std::max<int64_t>(1, std::min<int64_t>(want, std::min<int64_t>(cap, 4096))));
 }
 
+size_t vjp_rows_bytes(const Shape &S, int64_t B, int chunks) { return size_t(B) * chunks * nacc_of(S.D) * 16 + 256; }
+
+size_t vjp_min_ws_bytes(const Shape &S, int64_t B) { return vjp_rows_bytes(S, B, vjp_chunks_min_ws(S.N, B)); }
+
+// Blocks per triple and row group over `points` points: at least two points
+// per thread, and no more blocks than are resident at a time (D <= 4: four
+// per CU, D <= 6: two, D >= 7: one per row group), so that all of them advance
+// through the lattice together; a multiple of the XCD count.
+int vjp_chunks(int D, int64_t points, int64_t B) {
+    const int64_t cap = std::max<int64_t>(1, (D <= 4 ? 1024 : (D <= 6 ? 512 : 256)) / std::max<int64_t>(B, 1));
+    int64_t n = std::max<int64_t>(1, std::min<int64_t>((points + 511) / 512, cap));
+    if (n > MM_XCDS) n -= n % MM_XCDS;
+    return int(n);
+}
+
 size_t vjp_ws_bytes(const Shape &S, int64_t B) {
-    return size_t(B) * vjp_chunks(S.N, B) * nacc_of(S.D) * 16 + 256;
+    return std::max(vjp_min_ws_bytes(S, B), vjp_rows_bytes(S, B, vjp_chunks(S.D, S.N, B)));
 }
 
-// VJP of one stored lattice slab by slab (all row groups of a slab in one
-// launch, so each slab is fetched about once rather than once per group):
-// taken for D >= 5 (two or three row groups) when the slabs are large.
-bool vjp_by_slabs(const Shape &S, int64_t B) { return B == 1 && S.D >= 5 && S.st[0] >= (int64_t(1) << 16); }
-
-int launch_vjp_slabs(const Shape &S, const double *G, const double *g, const double *c, double *dA, double *db, double *dc, void *ws,
-                     const DevState *ds, hipStream_t s);
-
-int launch_vjp_sums(const Shape &S, int64_t B, const double *G, const double *g, const double *c, double *dA, double *db, double *dc,
-                    void *ws, size_t ws_bytes, const DevState *ds, hipStream_t s);
-
-// The stored lattice's VJP, then the non-finite fix-up (fix = false when the
-// caller launches its own).
-int launch_vjp(const Shape &S, int64_t B, const double *G, const double *g, const double *c, double *dA, double *db, double *dc,
-               void *ws, size_t ws_bytes, const DevState *ds, hipStream_t s, bool fix = true) {
-    int rc = launch_vjp_sums(S, B, G, g, c, dA, db, dc, ws, ws_bytes, ds, s);
-    if (rc || !fix) return rc;
-    return launch_fixup(S, B, nullptr, nullptr, c, g, const_cast<double *>(G), dA, db, dc, nullptr, false, true, ds, s);
+template <int D, bool SLAB, bool FWD>
+void launch_vjp_kernel_t(const VjpArgs &a, int64_t B, hipStream_t s) {
+    const dim3 grid(unsigned(a.nchunk * RowSplit<D>::NG), unsigned(B));
+    if (a.smax <= VJP_LDS_SQ)
+        hipLaunchKernelGGL((vjp_kernel<D, SLAB, FWD, true>), grid, dim3(256), size_t(a.smax + 2) * 8, s, a);
+    else
+        hipLaunchKernelGGL((vjp_kernel<D, SLAB, FWD, false>), grid, dim3(256), 0, s, a);
 }
 
-int launch_vjp_sums(const Shape &S, int64_t B, const double *G, const double *g, const double *c, double *dA, double *db, double *dc,
-                    void *ws, size_t ws_bytes, const DevState *ds, hipStream_t s) {
-    if (!ws || ws_bytes < vjp_ws_bytes(S, B))
-        return fail(MM_ERR_WORKSPACE, "VJP workspace of %zu bytes needed, %zu given", vjp_ws_bytes(S, B), ws_bytes);
-    if (vjp_by_slabs(S, B)) return launch_vjp_slabs(S, G, g, c, dA, db, dc, ws, ds, s);
+int launch_finalize(int D, int64_t B, const double2 *partial, int nchunk, const double *c, double *dA, double *db, double *dc, bool conj,
+                    hipStream_t s);
+
+// Fields common to the whole-lattice and the slab-by-slab VJP.
+VjpArgs vjp_args(const Shape &S, void *partial, int nchunk, int64_t points, bool conj, const DevState *ds) {
     VjpArgs a;
+    memset(&a, 0, sizeof(a));
     a.g = geom_of(S);
+    a.partial = reinterpret_cast<double2 *>(partial);
+    a.sq = ds->sq;
+    a.rsq = ds->rsq;
+    a.gsign = conj ? -1.0 : 1.0;
+    a.nchunk = nchunk;
+    a.visit = int(std::max<int64_t>(1, std::min<int64_t>(4, (points + int64_t(nchunk) * 256 - 1) / (int64_t(nchunk) * 256))));
+    a.smax = *std::max_element(S.s, S.s + S.D);
+    return a;
+}
+
+// The stored lattices' VJP (one launch and the finalize).  conj: of the
+// conjugated cotangent, the results conjugated (torch's convention).
+int launch_vjp_sums(const Shape &S, int64_t B, const double *G, const double *g, const double *c, double *dA, double *db, double *dc,
+                    void *ws, size_t ws_bytes, bool conj, const DevState *ds, hipStream_t s) {
+    if (!ws || ws_bytes < vjp_min_ws_bytes(S, B))
+        return fail(MM_ERR_WORKSPACE, "VJP workspace of %zu bytes needed, %zu given", vjp_ws_bytes(S, B), ws_bytes);
+    int nchunk = vjp_chunks(S.D, S.N, B);
+    if (ws_bytes < vjp_rows_bytes(S, B, nchunk)) nchunk = std::min(nchunk, vjp_chunks_min_ws(S.N, B));
+    VjpArgs a = vjp_args(S, ws, nchunk, S.N, conj, ds);
     a.G = reinterpret_cast<const double2 *>(G);
     a.gg = reinterpret_cast<const double2 *>(g);
-    a.partial = reinterpret_cast<double2 *>(ws);
-    a.sq = ds->sq;
-    a.nchunks = vjp_chunks(S.N, B);
-    dim3 grid(a.nchunks, unsigned(B));
-    const double2 *c2 = reinterpret_cast<const double2 *>(c);
-    double2 *dA2 = reinterpret_cast<double2 *>(dA), *db2 = reinterpret_cast<double2 *>(db), *dc2 = reinterpret_cast<double2 *>(dc);
     switch (S.D) {
-#define CASE(DD)                                                                                               \
-    case DD:                                                                                                   \
-        launch_vjp_groups<DD>(a, grid, s);                                                                     \
-        LAUNCH_CHECK("vjp_kernel");                                                                            \
-        hipLaunchKernelGGL((vjp_finalize<DD>), dim3(unsigned(B)), dim3(finalize_threads(B)), 0, s, a.partial, a.nchunks, c2, dA2, db2, dc2); \
-        LAUNCH_CHECK("vjp_finalize");                                                                          \
-        break;
+#define CASE(DD) \
+    case DD: launch_vjp_kernel_t<DD, false, false>(a, B, s); break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
         default:
             return fail(MM_ERR_INVALID, "bad D");
     }
-    return MM_OK;
+    LAUNCH_CHECK("vjp_kernel");
+    return launch_finalize(S.D, B, a.partial, nchunk, c, dA, db, dc, conj, s);
 }
 
-// One launch of slab_fused_kernel for level-0 slab m: the VJP terms of slab m
-// (cur, p1, p2 = slabs m, m-1, m-2) added into nblk partial rows, and, when
-// nxt is not NULL, the forward of slab m + 1 into nxt.
-template <int D>
-void launch_slab_fused_t(const SlabVjpArgs &v, const Slab0Args &f, bool fwd, int nblk, hipStream_t s) {
-    constexpr int NG = RowSplit<D>::NG;
-    if (fwd)
-        hipLaunchKernelGGL((slab_fused_kernel<D, true>), dim3(unsigned(nblk * (NG + 1))), dim3(256), 0, s, v, f);
-    else
-        hipLaunchKernelGGL((slab_fused_kernel<D, false>), dim3(unsigned(nblk * NG)), dim3(256), 0, s, v, f);
+// The stored lattices' VJP, then the non-finite fix-up (fix = false when the
+// caller launches its own).
+int launch_vjp(const Shape &S, int64_t B, const double *G, const double *g, const double *c, double *dA, double *db, double *dc,
+               void *ws, size_t ws_bytes, bool conj, const DevState *ds, hipStream_t s, bool fix = true) {
+    int rc = launch_vjp_sums(S, B, G, g, c, dA, db, dc, ws, ws_bytes, conj, ds, s);
+    if (rc || !fix) return rc;
+    return launch_fixup(S, B, nullptr, nullptr, c, g, const_cast<double *>(G), dA, db, dc, nullptr, false, true, ds, s, false, conj);
 }
 
-int launch_slab_fused(const Shape &S, const double *A, const double *b, const double2 *cur, const double2 *p1, const double2 *p2,
-                      const double2 *gg, double2 *nxt, double2 *partial, int nblk, int m, const DevState *ds, hipStream_t s) {
-    SlabVjpArgs v;
-    v.g = geom_of(S);
-    v.cur = cur;
-    v.p1 = p1;
-    v.p2 = p2;
-    v.gg = gg;
-    v.partial = partial;
-    v.sq = ds->sq;
-    v.m = m;
-    Slab0Args f;
-    f.g = v.g;
-    f.A = reinterpret_cast<const double2 *>(A);
-    f.b = reinterpret_cast<const double2 *>(b);
-    f.p1 = cur;
-    f.p2 = p1;
-    f.cur = nxt;
-    f.sq = ds->sq;
-    f.rsq = ds->rsq;
-    f.m = m + 1;
-    switch (S.D) {
-#define CASE(DD) \
-    case DD: launch_slab_fused_t<DD>(v, f, nxt != nullptr, nblk, s); break;
-        CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+// Level 0 slab by slab: the VJP terms of slab m and, for m + 1 < shape[0], the
+// forward of slab m + 1 into `slab(m + 1)`, one launch per slab, partial sums
+// in nchunk rows; then the finalize.  slab(m): address of slab m; slabs m - 1
+// to m + 1 must not share memory.
+template <class SlabAt>
+int launch_level0_vjp(const Shape &S, const double *A, const double *b, const double *c, const double *g, SlabAt slab, double *dA,
+                      double *db, double *dc, void *partial, int nchunk, const DevState *ds, hipStream_t s) {
+    const int64_t S0 = S.st[0];
+    VjpArgs a = vjp_args(S, partial, nchunk, S0, false, ds);
+    a.A = reinterpret_cast<const double2 *>(A);
+    a.b = reinterpret_cast<const double2 *>(b);
+    const double2 *g2 = reinterpret_cast<const double2 *>(g);
+    for (int m = 0; m < S.s[0]; ++m) {
+        const bool last = m + 1 == S.s[0];
+        a.m = m;
+        a.G = slab(m);
+        a.Gdn = m ? slab(m - 1) : a.G;
+        a.gg = g2 + int64_t(m) * S0;
+        a.gup = last ? a.gg : a.gg + S0;
+        a.nxt = last ? nullptr : slab(m + 1);
+        switch (S.D) {
+#define CASE(DD)                                                  \
+    case DD:                                                      \
+        if (last)                                                 \
+            launch_vjp_kernel_t<DD, true, false>(a, 1, s);        \
+        else                                                      \
+            launch_vjp_kernel_t<DD, true, true>(a, 1, s);         \
+        break;
+            CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
-        default:
-            return fail(MM_ERR_INVALID, "bad D");
+            default:
+                return fail(MM_ERR_INVALID, "bad D");
+        }
+        LAUNCH_CHECK("vjp_kernel");
     }
-    LAUNCH_CHECK("slab_fused_kernel");
-    return MM_OK;
+    return launch_finalize(S.D, 1, a.partial, nchunk, c, dA, db, dc, false, s);
 }
 
-// Blocks per row group of a slab_fused_kernel launch over slabs of S0 points.
-int slab_blocks(int64_t S0, const DevState *ds) {
-    return int(std::max<int64_t>(1, std::min<int64_t>((S0 + 1023) / 1024, int64_t(ds->num_cu) * 8)));
-}
-
-// Sum nblk partial rows of one triple and finish (symmetrise, dc = sum / c).
-int launch_finalize(int D, const double2 *partial, int nblk, const double *c, double *dA, double *db, double *dc, hipStream_t s) {
+// Sum the nchunk partial rows of every triple and finish (symmetrise, dc = sum / c).
+int launch_finalize(int D, int64_t B, const double2 *partial, int nchunk, const double *c, double *dA, double *db, double *dc, bool conj,
+                    hipStream_t s) {
     const double2 *c2 = reinterpret_cast<const double2 *>(c);
     double2 *dA2 = reinterpret_cast<double2 *>(dA), *db2 = reinterpret_cast<double2 *>(db), *dc2 = reinterpret_cast<double2 *>(dc);
+    const double gs = conj ? -1.0 : 1.0;
     switch (D) {
-#define CASE(DD) \
-    case DD: hipLaunchKernelGGL((vjp_finalize<DD>), dim3(1), dim3(finalize_threads(1)), 0, s, partial, nblk, c2, dA2, db2, dc2); break;
+#define CASE(DD)                                                                                                                    \
+    case DD:                                                                                                                        \
+        hipLaunchKernelGGL((vjp_finalize<DD>), dim3(unsigned(B)), dim3(finalize_threads(B)), 0, s, partial, nchunk, c2, dA2, db2, dc2, \
+                           gs);                                                                                                     \
+        break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
         default:
@@ -837,25 +849,6 @@ int launch_stable(const Shape &S, int64_t B, const double *A, const double *b, c
     return launch_fixup(S, B, A, b, c, nullptr, G, nullptr, nullptr, nullptr, nf, true, false, ds, s, true);
 }
 
-// The stored lattice's VJP, one slab_fused_kernel launch per level-0 slab
-// (no forward role).  The workspace holds at least slab_blocks rows.
-int launch_vjp_slabs(const Shape &S, const double *G, const double *g, const double *c, double *dA, double *db, double *dc, void *ws,
-                     const DevState *ds, hipStream_t s) {
-    const int64_t S0 = S.st[0];
-    const int nblk = std::min(slab_blocks(S0, ds), vjp_chunks(S.N, 1));
-    double2 *partial = reinterpret_cast<double2 *>(ws);
-    hipLaunchKernelGGL(zero_c128_kernel, dim3(64), dim3(256), 0, s, partial, int64_t(nblk) * nacc_of(S.D));
-    LAUNCH_CHECK("zero_c128_kernel");
-    const double2 *G2 = reinterpret_cast<const double2 *>(G), *g2 = reinterpret_cast<const double2 *>(g);
-    for (int m = 0; m < S.s[0]; ++m) {
-        const double2 *cur = G2 + int64_t(m) * S0;
-        const int rc = launch_slab_fused(S, nullptr, nullptr, cur, m >= 1 ? cur - S0 : cur, m >= 2 ? cur - 2 * S0 : cur, g2 + int64_t(m) * S0,
-                                         nullptr, partial, nblk, m, ds, s);
-        if (rc) return rc;
-    }
-    return launch_finalize(S.D, partial, nblk, c, dA, db, dc, s);
-}
-
 // ------------------------------------------------------------ vanilla paths
 
 // Workspace of one vanilla forward (+ fused VJP when `fused`).
@@ -880,9 +873,6 @@ size_t fwd_ws_bytes(const Shape &S, bool fused, const DevState *ds) {
     if (top == 0 && !spread_single(S, true, 1, ds, &Tf)) return 0;
     return vjp_ws_bytes(S, 1);
 }
-
-int window_slab0(const Shape &S, const double *A, const double *b, double2 *cur, double2 *p1, double2 *p2, int m,
-                 const DevState *ds, hipStream_t s);
 
 // Forward of B triples sharing shape S (uniform strides); fused adds the VJP.
 int vanilla_uniform(const Shape &S, int64_t B, const double *A, const double *b, const double *c, const double *g, double *G,
@@ -914,7 +904,7 @@ int vanilla_uniform(const Shape &S, int64_t B, const double *A, const double *b,
     // a single triple with large level-0 slabs over all CUs (spread_single);
     // with the VJP only when the caller gave the VJP workspace for it
     int Tf = 64;
-    const bool spread = top == 0 && spread_single(S, fused, B, ds, &Tf) && (!fused || (ws && ws_bytes >= vjp_ws_bytes(S, 1)));
+    const bool spread = top == 0 && spread_single(S, fused, B, ds, &Tf) && (!fused || (ws && ws_bytes >= vjp_min_ws_bytes(S, 1)));
     if (top == 0 && !spread) {
         a.tmpl = make_job(S, 0, KIND_BLOCK);
         int64_t shmem = lds_bytes(S, 0, fused, T / MM_WAVE, kernel_dmax(S.D));
@@ -929,7 +919,7 @@ int vanilla_uniform(const Shape &S, int64_t B, const double *A, const double *b,
     } else {
         top = choose_top(S, false, ds->max_lds, lds_maxt(S.D, false), &T);
     }
-    if (fused && (!ws || ws_bytes < vjp_ws_bytes(S, B)))
+    if (fused && (!ws || ws_bytes < vjp_min_ws_bytes(S, B)))
         return fail(MM_ERR_WORKSPACE, "fused workspace of %zu bytes needed, %zu given", vjp_ws_bytes(S, B), ws_bytes);
     int *nf = nullptr;
     {
@@ -951,43 +941,28 @@ int vanilla_uniform(const Shape &S, int64_t B, const double *A, const double *b,
         sa.sq = ds->sq;
         sa.rsq = ds->rsq;
         sa.nf = nf;
-        // with the VJP of a single triple above 512 MB, level 0 alternates the
-        // VJP terms of slab m (every row group in one launch) with the forward
-        // of slab m + 1, so that each slab is read while it is still in the
-        // caches; below that, the forward (two slabs per launch) then one VJP
-        // pass take fewer launches and measured faster ((60,)^4, 207 MB: 0.82
-        // against 1.12 ms; (10,)^8, 1.6 GB: 6.76 ms interleaved against 6.9)
+        // with the VJP of a single triple above 512 MB, each level-0 launch
+        // takes the VJP terms of slab m and the forward of slab m + 1 from the
+        // same loads; below that, the forward (two slabs per launch) then one
+        // VJP pass take fewer launches
         const bool fuse_level0 = fused && B == 1 && S.N * 16 > (int64_t(512) << 20);
         for (int d = top - 1; d >= (fuse_level0 ? 1 : 0); --d) {
             rc = launch_level(sa, S, d, ds, s);
             if (rc) return rc;
         }
         if (fuse_level0) {
-            const int64_t S0 = S.st[0];
-            const int nblk = std::min(slab_blocks(S0, ds), vjp_chunks(S.N, 1));
-            double2 *partial = reinterpret_cast<double2 *>(ws);
-            hipLaunchKernelGGL(zero_c128_kernel, dim3(64), dim3(256), 0, s, partial, int64_t(nblk) * nacc_of(S.D));
-            LAUNCH_CHECK("zero_c128_kernel");
             double2 *G2 = sa.G;
-            const double2 *g2 = reinterpret_cast<const double2 *>(g) + t * a.ug;
-            for (int m = 0; m < S.s[0]; ++m) {
-                double2 *cur = G2 + int64_t(m) * S0;
-                rc = launch_slab_fused(S, A + 2 * t * a.ua, b + 2 * t * a.ub, cur, m >= 1 ? cur - S0 : cur, m >= 2 ? cur - 2 * S0 : cur,
-                                       g2 + int64_t(m) * S0, nullptr, partial, nblk, m, ds, s);
-                if (rc) return rc;
-                if (m + 1 < S.s[0]) {
-                    rc = window_slab0(S, A + 2 * t * a.ua, b + 2 * t * a.ub, cur + S0, cur, m >= 1 ? cur - S0 : cur, m + 1, ds, s);
-                    if (rc) return rc;
-                }
-            }
-            rc = launch_finalize(S.D, partial, nblk, c + 2 * t, dA + 2 * t * a.ua, db + 2 * t * a.ub, dc + 2 * t, s);
+            const int nchunk = std::min(vjp_chunks(S.D, S.st[0], 1), vjp_chunks_min_ws(S.N, 1));
+            rc = launch_level0_vjp(S, A + 2 * t * a.ua, b + 2 * t * a.ub, c + 2 * t, g + 2 * t * a.ug,
+                                   [G2, &S](int m) { return G2 + int64_t(m) * S.st[0]; }, dA + 2 * t * a.ua, db + 2 * t * a.ub, dc + 2 * t,
+                                   ws, nchunk, ds, s);
             if (rc) return rc;
             return launch_fixup(S, 1, A + 2 * t * a.ua, b + 2 * t * a.ub, c + 2 * t, g + 2 * t * a.ug, G + 2 * t * a.ug, dA + 2 * t * a.ua,
                                 db + 2 * t * a.ub, dc + 2 * t, nf, true, true, ds, s);
         }
     }
     if (fused) {
-        const int rc = launch_vjp(S, B, G, g, c, dA, db, dc, ws, ws_bytes, ds, s, false);
+        const int rc = launch_vjp(S, B, G, g, c, dA, db, dc, ws, ws_bytes, false, ds, s, false);
         if (rc) return rc;
     }
     return launch_fixup(S, B, A, b, c, g, G, dA, db, dc, nf, true, fused, ds, s);
@@ -1003,8 +978,10 @@ int vanilla_uniform(const Shape &S, int64_t B, const double *A, const double *b,
 // most 64 MB, and those whose slabs fit in LDS, take the fused sweep with a
 // full G in the workspace (recompute_whole).
 
-int recompute_blocks(const Shape &S, const DevState *ds) { return slab_blocks(S.st[0], ds); }
-
+// Partial rows of the window's workspace.
+int recompute_rows(const Shape &S, const DevState *ds) {
+    return int(std::max<int64_t>(1, std::min<int64_t>((S.st[0] + 1023) / 1024, int64_t(ds->num_cu) * 8)));
+}
 
 // Lattices held whole in the workspace instead of the window: those whose
 // fused slabs fit in LDS, and any of at most 64 MB (the window's slab-by-slab
@@ -1018,10 +995,12 @@ bool recompute_whole(const Shape &S, const DevState *ds, bool *vjp_ws) {
     return whole;
 }
 
-size_t recompute_ws_bytes(const Shape &S, const DevState *ds) {
+// Workspace of the recompute VJP: what the call asks for, or the least it takes.
+size_t recompute_ws_bytes(const Shape &S, const DevState *ds, bool least) {
     bool vjp_ws = false;
-    if (recompute_whole(S, ds, &vjp_ws)) return align256(size_t(S.N) * 16) + (vjp_ws ? vjp_ws_bytes(S, 1) : 0);
-    return 3 * align256(size_t(S.st[0]) * 16) + size_t(recompute_blocks(S, ds)) * nacc_of(S.D) * 16 + 256;
+    if (recompute_whole(S, ds, &vjp_ws))
+        return align256(size_t(S.N) * 16) + (vjp_ws ? (least ? vjp_min_ws_bytes(S, 1) : vjp_ws_bytes(S, 1)) : 0);
+    return 3 * align256(size_t(S.st[0]) * 16) + size_t(recompute_rows(S, ds)) * nacc_of(S.D) * 16 + 256;
 }
 
 // The face {k_0 = 0} of the lattice into `face` (stride[0] entries): the LDS
@@ -1089,7 +1068,7 @@ int window_slab0(const Shape &S, const double *A, const double *b, double2 *cur,
 
 int vjp_recompute(const Shape &S, const double *A, const double *b, const double *c, const double *g, double *dA, double *db,
                   double *dc, void *ws, size_t ws_bytes, const DevState *ds, hipStream_t s) {
-    const size_t need = recompute_ws_bytes(S, ds);
+    const size_t need = recompute_ws_bytes(S, ds, true);
     if (!ws || ws_bytes < need) return fail(MM_ERR_WORKSPACE, "recompute workspace of %zu bytes needed, %zu given", need, ws_bytes);
     bool vjp_ws = false;
     if (recompute_whole(S, ds, &vjp_ws)) {
@@ -1098,35 +1077,19 @@ int vjp_recompute(const Shape &S, const double *A, const double *b, const double
                                ws_bytes - gb, ds, s);
     }
 
-    // three slabs: slab m + 1 is computed into the slot of slab m - 2 once the
-    // VJP terms of slab m (the last to read slab m - 2) are launched
+    // three slabs: the launch of slab m reads slabs m and m - 1 and writes slab m + 1
     const size_t slab_bytes = align256(size_t(S.st[0]) * 16);
     char *base = reinterpret_cast<char *>(ws);
     double2 *slot[3];
     for (int i = 0; i < 3; ++i) slot[i] = reinterpret_cast<double2 *>(base + i * slab_bytes);
     double2 *partial = reinterpret_cast<double2 *>(base + 3 * slab_bytes);
-    const int nblk = recompute_blocks(S, ds);
-    const int NA = nacc_of(S.D);
-    hipLaunchKernelGGL(zero_c128_kernel, dim3(64), dim3(256), 0, s, partial, int64_t(nblk) * NA);
-    LAUNCH_CHECK("zero_c128_kernel");
 
     // 1. the face {k_0 = 0} into slot 0
     int rc = window_face(S, A, b, c, slot[0], ds, s);
     if (rc) return rc;
-    // 2. level 0: the VJP terms of slab m (every row group in one launch), then slab m + 1
-    const int64_t S0 = S.st[0];
-    for (int m = 0; m < S.s[0]; ++m) {
-        double2 *cur = slot[m % 3];
-        rc = launch_slab_fused(S, A, b, cur, m >= 1 ? slot[(m + 2) % 3] : cur, m >= 2 ? slot[(m + 1) % 3] : cur,
-                               reinterpret_cast<const double2 *>(g) + int64_t(m) * S0, nullptr, partial, nblk, m, ds, s);
-        if (rc) return rc;
-        if (m + 1 < S.s[0]) {
-            rc = window_slab0(S, A, b, slot[(m + 1) % 3], cur, m >= 1 ? slot[(m + 2) % 3] : cur, m + 1, ds, s);
-            if (rc) return rc;
-        }
-    }
-    // 3. sum the block partials and finish (symmetrise, dc = sum / c)
-    return launch_finalize(S.D, partial, nblk, c, dA, db, dc, s);
+    // 2. level 0: the VJP terms of slab m with slab m + 1, then the sums' end
+    return launch_level0_vjp(S, A, b, c, g, [&slot](int m) { return slot[m % 3]; }, dA, db, dc, partial,
+                             std::min(vjp_chunks(S.D, S.st[0], 1), recompute_rows(S, ds)), ds, s);
 }
 
 // ------------------------------------------------------------------- plans
@@ -1343,7 +1306,32 @@ int mm_hermite_batch_vjp(const double *G, const double *c, const double *dLdG, i
     DevState *ds = nullptr;
     rc = device_state(&ds);
     if (rc) return rc;
-    return launch_vjp(S, B, G, dLdG, c, dA, db, dc, workspace, ws_bytes, ds, reinterpret_cast<hipStream_t>(stream));
+    return launch_vjp(S, B, G, dLdG, c, dA, db, dc, workspace, ws_bytes, false, ds, reinterpret_cast<hipStream_t>(stream));
+}
+
+int mm_hermite_batch_vjp_conj(const double *G, const double *c, const double *grad, int64_t B, const int64_t *shape, int D, double *dA,
+                              double *db, double *dc, void *workspace, size_t ws_bytes, void *stream) {
+    Shape S;
+    int rc = make_shape(shape, D, &S);
+    if (rc) return rc;
+    if (B < 0) return fail(MM_ERR_INVALID, "negative batch size");
+    if (B == 0) return MM_OK;
+    if (B > 65535) return fail(MM_ERR_UNSUPPORTED, "batch of %lld > 65535 triples", (long long)B);
+    if (!G || !c || !grad || !dA || !db || !dc) return fail(MM_ERR_INVALID, "NULL array pointer");
+    DevState *ds = nullptr;
+    rc = device_state(&ds);
+    if (rc) return rc;
+    return launch_vjp(S, B, G, grad, c, dA, db, dc, workspace, ws_bytes, true, ds, reinterpret_cast<hipStream_t>(stream));
+}
+
+int mm_conj_triple(const double *A, int64_t nA, const double *b, int64_t nb, const double *c, double *out, void *stream) {
+    if (!A || !b || !c || !out) return fail(MM_ERR_INVALID, "NULL array pointer");
+    if (nA < 1 || nb < 1 || nA > 4096 || nb > 64) return fail(MM_ERR_INVALID, "nA=%lld, nb=%lld entries", (long long)nA, (long long)nb);
+    hipLaunchKernelGGL(conj_triple_kernel, dim3(1), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const double2 *>(A),
+                       int(nA), reinterpret_cast<const double2 *>(b), int(nb), reinterpret_cast<const double2 *>(c),
+                       reinterpret_cast<double2 *>(out));
+    LAUNCH_CHECK("conj_triple_kernel");
+    return MM_OK;
 }
 
 int mm_hermite_batch_vjp_static(const double *G, const double *c, const double *dLdG, int64_t B, const int64_t *shape, int D,
@@ -1355,7 +1343,7 @@ int mm_hermite_batch_vjp_static(const double *G, const double *c, const double *
     if (B == 0) return MM_OK;
     if (B > 65535) return fail(MM_ERR_UNSUPPORTED, "batch of %lld > 65535 triples", (long long)B);
     if (!G || !c || !dLdG || !dA || !db || !dc) return fail(MM_ERR_INVALID, "NULL array pointer");
-    const size_t need = vjp_ws_bytes(S, B);
+    const size_t need = vjp_min_ws_bytes(S, B);
     if (need > size_t(MM_STATIC_SCRATCH_BYTES))
         return fail(MM_ERR_UNSUPPORTED, "this VJP needs %zu bytes of scratch, above the static buffer's %zu; use mm_hermite_batch_vjp",
                     need, size_t(MM_STATIC_SCRATCH_BYTES));
@@ -1366,7 +1354,7 @@ int mm_hermite_batch_vjp_static(const double *G, const double *c, const double *
     DevState *ds = nullptr;
     rc = device_state(&ds);
     if (rc) return rc;
-    return launch_vjp(S, B, G, dLdG, c, dA, db, dc, ws, size_t(MM_STATIC_SCRATCH_BYTES), ds, reinterpret_cast<hipStream_t>(stream));
+    return launch_vjp(S, B, G, dLdG, c, dA, db, dc, ws, size_t(MM_STATIC_SCRATCH_BYTES), false, ds, reinterpret_cast<hipStream_t>(stream));
 }
 
 size_t mm_hermite_fused_workspace(const int64_t *shape, int D) {
@@ -1610,7 +1598,7 @@ size_t mm_hermite_vjp_recompute_workspace(const int64_t *shape, int D) {
     if (make_shape(shape, D, &S)) return 0;
     DevState *ds = nullptr;
     if (device_state(&ds)) return 0;
-    return recompute_ws_bytes(S, ds);
+    return recompute_ws_bytes(S, ds, false);
 }
 
 int mm_hermite_vjp_recompute(const double *A, const double *b, const double *c, const double *dLdG, const int64_t *shape, int D,

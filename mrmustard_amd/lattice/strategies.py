@@ -14,6 +14,8 @@ ABI of libmmhip.so on the current stream:
   equals the two calls in sequence).
 - ``vanilla_vjp_recompute_hip``: the VJP from (A, b, c) without G, recomputing
   the lattice slab by slab in a bounded window.
+- ``vanilla_vjp_grad_hip``: the VJP in torch's gradient convention;
+  ``conj_triple`` serves the VJPs that recompute the forward.
 - ``binomial_hip``           <- binomial.py:30-74  ``binomial`` (fill by weight,
   stop on the squared norm).
 
@@ -23,6 +25,7 @@ conjugated, and dA is returned symmetrised, (M + M^T)/2.
 
 from __future__ import annotations
 
+import cmath
 import ctypes
 import math as pymath
 
@@ -33,6 +36,7 @@ from .. import _lib
 
 __all__ = [
     "binomial_hip",
+    "conj_triple",
     "stable_hip",
     "vanilla_vjp_recompute_hip",
     "vanilla_batch_fused_hip",
@@ -40,6 +44,7 @@ __all__ = [
     "vanilla_batch_vjp_hip",
     "vanilla_fused_hip",
     "vanilla_hip",
+    "vanilla_vjp_grad_hip",
     "vanilla_vjp_hip",
 ]
 
@@ -195,6 +200,45 @@ def vanilla_batch_vjp_hip(G, c, dLdG):
     return dA, db, dc
 
 
+def vanilla_vjp_grad_hip(G, c, grad, batched: bool = False):
+    """The VJP in torch's convention: for ``grad`` = dL/d(conj G), the tensors
+    conj(VJP(conj(grad))) that torch expects, of one lattice or of a batch.  The
+    kernel reads ``grad`` and writes its results conjugated, so no conjugated
+    copy is made."""
+    L = _lib.load()
+    G, g, c = as_device_c128(G), as_device_c128(grad), as_device_c128(c).reshape(-1)
+    if tuple(g.shape) != tuple(G.shape):
+        raise ValueError("the gradient must have the shape of G")
+    lead = (int(G.shape[0]),) if batched else ()
+    B = lead[0] if batched else 1
+    D = G.dim() - len(lead)
+    s = _shape_arr(G.shape[len(lead):])
+    dA = torch.empty((*lead, D, D), dtype=C128, device=G.device)
+    db = torch.empty((*lead, D), dtype=C128, device=G.device)
+    dc = torch.empty(lead, dtype=C128, device=G.device)
+    if B == 0:
+        return dA, db, dc
+    ws = _workspace(L.mm_hermite_batch_vjp_workspace(B, s.ctypes.data, D))
+    rc = L.mm_hermite_batch_vjp_conj(
+        _ptr(G), _ptr(c), _ptr(g), B, s.ctypes.data, D, _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws), 0 if ws is None else ws.numel(),
+        _stream(),
+    )
+    _lib.check(rc, "mm_hermite_batch_vjp_conj")
+    return dA, db, dc
+
+
+def conj_triple(A, b, c):
+    """(conj A, conj b, conj c) in one launch.  A VJP in torch's convention,
+    conj(VJP(A, b, c; conj(grad))), equals VJP(conj A, conj b, conj c; grad):
+    the lattice of the conjugated triple is the conjugated lattice."""
+    A, b, c = as_device_c128(A), as_device_c128(b), as_device_c128(c)
+    nA, nb = A.numel(), b.numel()
+    buf = torch.empty(nA + nb + 1, dtype=C128, device=A.device)
+    rc = _lib.load().mm_conj_triple(_ptr(A), nA, _ptr(b), nb, _ptr(c), _ptr(buf), _stream())
+    _lib.check(rc, "mm_conj_triple")
+    return buf[:nA].view(A.shape), buf[nA : nA + nb].view(b.shape), buf[nA + nb :].view(c.shape)
+
+
 def vanilla_fused_hip(shape, A, b, c, dLdG, out=None):
     """G and its VJP in one sweep: (G, dA, db, dc)."""
     L = _lib.load()
@@ -268,7 +312,7 @@ def vanilla_vjp_recompute_hip(shape, A, b, c, dLdG):
         0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_vjp_recompute")
-    if not bool(torch.isfinite(dc)):
+    if not cmath.isfinite(dc.item()):
         return vanilla_vjp_hip(vanilla_hip(shape, A, b, c), c, g)
     return dA, db, dc
 

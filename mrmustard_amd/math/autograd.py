@@ -8,8 +8,10 @@ exactly as ``hermite_renormalized_jax_bwd`` always calls ``vanilla_vjp_numba``.
 Convention.  The reference VJP is holomorphic: it returns sum_k g_k dG_k/dtheta
 for the cotangent g, unconjugated.  torch hands a backward function
 grad = dL/d(conj G) and expects dL/d(conj theta), which for a holomorphic map
-is conj( sum_k conj(grad_k) dG_k/dtheta ).  So the backward conjugates the
-incoming gradient, runs the reference VJP, and conjugates the result.
+is conj( sum_k conj(grad_k) dG_k/dtheta ).  The stored-lattice VJP reads the
+gradient and writes its results conjugated; the VJPs that recompute the
+forward run it at (conj A, conj b, conj c) with the gradient as it is, which is
+the same number: no conjugated copy of a lattice-sized gradient is made.
 """
 
 from __future__ import annotations
@@ -32,14 +34,8 @@ class HermiteRenormalized(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad):
         G, c = ctx.saved_tensors
-        dA, db, dc = st.vanilla_vjp_hip(G, c, grad.conj())
-        return (
-            dA.conj().resolve_conj().reshape(ctx.a_shape),
-            db.conj().resolve_conj().reshape(ctx.b_shape),
-            dc.conj().resolve_conj().reshape(ctx.c_shape),
-            None,
-            None,
-        )
+        dA, db, dc = st.vanilla_vjp_grad_hip(G, c, grad)
+        return dA.reshape(ctx.a_shape), db.reshape(ctx.b_shape), dc.reshape(ctx.c_shape), None, None
 
 
 class HermiteRenormalizedBatched(torch.autograd.Function):
@@ -55,14 +51,8 @@ class HermiteRenormalizedBatched(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad):
         G, c = ctx.saved_tensors
-        dA, db, dc = st.vanilla_batch_vjp_hip(G, c, grad.conj())
-        return (
-            dA.conj().resolve_conj().reshape(ctx.a_shape),
-            db.conj().resolve_conj().reshape(ctx.b_shape),
-            dc.conj().resolve_conj().reshape(ctx.c_shape),
-            None,
-            None,
-        )
+        dA, db, dc = st.vanilla_vjp_grad_hip(G, c, grad, batched=True)
+        return dA.reshape(ctx.a_shape), db.reshape(ctx.b_shape), dc.reshape(ctx.c_shape), None, None
 
 
 class HermiteRenormalizedRecompute(torch.autograd.Function):
@@ -88,17 +78,11 @@ class HermiteRenormalizedRecompute(torch.autograd.Function):
         A, b, c = ctx.saved_tensors
         if ctx.stable:
             G = st.stable_hip(ctx.shape, A, b, c)
-            dA, db, dc = st.vanilla_vjp_hip(G, c, grad.conj())
+            dA, db, dc = st.vanilla_vjp_grad_hip(G, c, grad)
             del G
         else:
-            dA, db, dc = st.vanilla_vjp_recompute_hip(ctx.shape, A, b, c, grad.conj())
-        return (
-            dA.conj().resolve_conj().reshape(A.shape),
-            db.conj().resolve_conj().reshape(b.shape),
-            dc.conj().resolve_conj().reshape(c.shape),
-            None,
-            None,
-        )
+            dA, db, dc = st.vanilla_vjp_recompute_hip(ctx.shape, *st.conj_triple(A, b, c), grad)
+        return dA.reshape(A.shape), db.reshape(b.shape), dc.reshape(c.shape), None, None
 
 
 class HermiteDiagonal(torch.autograd.Function):
@@ -121,14 +105,8 @@ class HermiteDiagonal(torch.autograd.Function):
         from ..lattice import compact_fock as cf
 
         A, B, c = ctx.saved_tensors
-        _, dA, dB, dc = cf.diagonal_vjp_hip(A, B, c, ctx.cutoffs, grad.conj().resolve_conj(), reordered=ctx.reordered)
-        return (
-            dA.conj().resolve_conj().reshape(A.shape),
-            dB.conj().resolve_conj().reshape(B.shape),
-            dc.conj().resolve_conj().reshape(c.shape),
-            None,
-            None,
-        )
+        _, dA, dB, dc = cf.diagonal_vjp_hip(*st.conj_triple(A, B, c), ctx.cutoffs, grad, reordered=ctx.reordered)
+        return dA.reshape(A.shape), dB.reshape(B.shape), dc.reshape(c.shape), None, None
 
 
 class HermiteLeftover(torch.autograd.Function):
@@ -152,12 +130,5 @@ class HermiteLeftover(torch.autograd.Function):
 
         A, b, c = ctx.saved_tensors
         o, pnr, reordered = ctx.args
-        _, dA, db, dc = cf.leftover_vjp_hip(A, b, c, o, pnr, grad.conj().resolve_conj(), reordered=reordered)
-        return (
-            dA.conj().resolve_conj().reshape(A.shape),
-            db.conj().resolve_conj().reshape(b.shape),
-            dc.conj().resolve_conj().reshape(c.shape),
-            None,
-            None,
-            None,
-        )
+        _, dA, db, dc = cf.leftover_vjp_hip(*st.conj_triple(A, b, c), o, pnr, grad, reordered=reordered)
+        return dA.reshape(A.shape), db.reshape(b.shape), dc.reshape(c.shape), None, None, None
