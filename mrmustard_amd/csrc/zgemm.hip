@@ -5,6 +5,41 @@
 
 using namespace mm;
 
+namespace {
+
+// Tile rows of zgemm_strip_kernel (16 RT rows each), or 0 for the 64 x 128
+// tiles of zgemm_mfma_kernel, which win by 2 to 5 % only where they fill
+// whole rounds of the chip (two workgroups per CU) with little padding:
+// 2048^3 1066 against 1121 us, but 1600^3 (325 tiles for 512 places) 829
+// against 640 us.  RT: all rows in one tile row (B read once) when the strips
+// alone keep every SIMD busy (100 x 10^6 x 100: 1584 us, 2024 with two tile
+// rows), else at most 4 for more workgroups (81 x 6561 x 81: 15.3 against 23.9 us).
+int strip_rt(int64_t M, int64_t N, int64_t batch, int num_cu) {
+    const int64_t big = ((M + 63) / 64) * ((N + ZG_BN - 1) / ZG_BN) * batch;
+    const int64_t rounds = (big + 2 * num_cu - 1) / (2 * num_cu);
+    if (M >= 512 && N >= 512 && double(M) * double(N) * double(batch) >= 0.9 * double(rounds) * 2.0 * num_cu * 64 * ZG_BN) return 0;
+    const int64_t mt = (M + 15) / 16;
+    if (mt <= 8 && (N * batch + 63) / 64 >= 4 * int64_t(num_cu)) return int(mt);
+    const int64_t gy = (mt + 3) / 4;
+    return int((mt + gy - 1) / gy);
+}
+
+// nz products of N columns each, or (cols > N) one with the columns of all.
+template <int RT>
+void launch_strip(const ZgemmArgs &a, int64_t nz, int64_t cols, hipStream_t s) {
+    const dim3 grid(unsigned((cols + 63) / 64), unsigned((a.M + 16 * RT - 1) / (16 * RT)), unsigned(nz));
+    if constexpr (RT <= 4) {
+        // the whole of K in one chunk: no second round trip to memory
+        if (a.K <= 16) {
+            hipLaunchKernelGGL((zgemm_strip_kernel<RT, 16>), grid, dim3(256), 0, s, a, cols);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((zgemm_strip_kernel<RT, ZG_BK>), grid, dim3(256), 0, s, a, cols);
+}
+
+}  // namespace
+
 extern "C" {
 
 int mm_zgemm_batched(const double *A, int64_t lda, int64_t sA, const double *B, int64_t ldb, int64_t sB, double *C, int64_t ldc,
@@ -15,10 +50,12 @@ int mm_zgemm_batched(const double *A, int64_t lda, int64_t sA, const double *B, 
     if (lda < K || ldb < N || ldc < N) return fail(MM_ERR_INVALID, "leading dimension smaller than the row length");
     if (sA < 0 || sB < 0 || sC < 0) return fail(MM_ERR_INVALID, "negative batch stride");
     if (batch > 1 && sC < (M - 1) * ldc + N) return fail(MM_ERR_INVALID, "the products of a batch overlap in C");
-    const bool tall = M > 64 && M <= 128;  // one 128-row tile covers M: B is read once
-    const int bm = tall ? 128 : 64;
-    const int64_t gx = (N + ZG_BN - 1) / ZG_BN, gy = (M + bm - 1) / bm;
-    if (gx > 0x7fffffff || gy > 65535) return fail(MM_ERR_UNSUPPORTED, "matrix too large for one launch");
+    const int64_t gx = (N + ZG_BN - 1) / ZG_BN, gy = (M + 63) / 64;
+    if (gx > 0x3fffffff || gy > 65535) return fail(MM_ERR_UNSUPPORTED, "matrix too large for one launch");
+    DevState *ds = nullptr;
+    const int rc = device_state(&ds);
+    if (rc) return rc;
+    const int rt = strip_rt(M, N, batch, ds->num_cu);
     ZgemmArgs a;
     a.M = M;
     a.N = N;
@@ -30,15 +67,23 @@ int mm_zgemm_batched(const double *A, int64_t lda, int64_t sA, const double *B, 
     a.sB = sB;
     a.sC = sC;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    for (int64_t b0 = 0; b0 < batch; b0 += 65535) {  // grid z holds at most 65535 products
-        const int64_t nz = std::min<int64_t>(65535, batch - b0);
+    // products that share A: one with all their columns, while grid x holds it
+    const bool flat = rt && sA == 0 && batch > 1 && N <= (int64_t(1) << 36) / batch;
+    const int64_t step = flat ? batch : 65535;  // grid z holds at most 65535 products
+    for (int64_t b0 = 0; b0 < batch; b0 += step) {
+        const int64_t nz = std::min<int64_t>(step, batch - b0);
         a.A = reinterpret_cast<const double2 *>(A) + b0 * sA;
         a.B = reinterpret_cast<const double2 *>(B) + b0 * sB;
         a.C = reinterpret_cast<double2 *>(C) + b0 * sC;
-        if (tall)
-            hipLaunchKernelGGL(zgemm_mfma_kernel<128>, dim3(unsigned(gx), unsigned(gy), unsigned(nz)), dim3(512), 0, s, a);
-        else
-            hipLaunchKernelGGL(zgemm_mfma_kernel<64>, dim3(unsigned(gx), unsigned(gy), unsigned(nz)), dim3(256), 0, s, a);
+        switch (rt) {
+            case 0:
+                hipLaunchKernelGGL(zgemm_mfma_kernel, dim3(unsigned(gx), unsigned(gy), unsigned(nz)), dim3(256), 0, s, a);
+                break;
+#define CASE(RT) \
+    case RT: launch_strip<RT>(a, flat ? 1 : nz, flat ? N * nz : N, s); break;
+                CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+#undef CASE
+        }
     }
     LAUNCH_CHECK("zgemm_mfma_kernel");
     return MM_OK;

@@ -6,8 +6,7 @@
 // backend_manager.py:526-548).  Row-major A (M x K, lda), B (K x N, ldb),
 // C (M x N, ldc), all interleaved (re, im) doubles.
 //
-// Tiling: a workgroup of 4 waves owns a 64 x 128 tile of C (8 waves, 128 x 128,
-// for 64 < M <= 128); wave w owns the 32 x 64 sub-tile (w / 2, w % 2), i.e.
+// Tiling: a workgroup of 4 waves owns a 64 x 128 tile of C; wave w owns the 32 x 64 sub-tile (w / 2, w % 2), i.e.
 // 2 x 4 tiles of 16 x 16, each with a
 // real and an imaginary accumulator (v_mfma_f64_16x16x4_f64, K = 4 per
 // instruction).  A complex product is four real ones:
@@ -37,11 +36,10 @@ struct ZgemmArgs {
 
 constexpr int ZG_BN = 128, ZG_BK = 8;
 
-// ZG_BM = 64 (4 waves, two workgroups per CU) in general; ZG_BM = 128 (8 waves,
-// one workgroup per CU, the same two waves per SIMD) when one tile row covers
-// M (64 < M <= 128), so that B is read once instead of twice.
-template <int ZG_BM>
-__global__ __launch_bounds__(ZG_BM * 4, ZG_BM == 64 ? 2 : 1) void zgemm_mfma_kernel(ZgemmArgs a) {
+// Two workgroups per CU.  Large products only (strip_plan): measured 64.5
+// TFLOP/s at 2048^3 and 65.4 at 4096^3, where zgemm_strip_kernel has 61.3 and 64.3.
+__global__ __launch_bounds__(256, 2) void zgemm_mfma_kernel(ZgemmArgs a) {
+    constexpr int ZG_BM = 64;
     constexpr int ZG_THREADS = ZG_BM * 4;
     a.A += int64_t(blockIdx.z) * a.sA;
     a.B += int64_t(blockIdx.z) * a.sB;
@@ -162,6 +160,121 @@ __global__ __launch_bounds__(ZG_BM * 4, ZG_BM == 64 ? 2 : 1) void zgemm_mfma_ker
                 const int64_t gn = n0 + wn + j * 16 + lr;
                 if (gm < a.M && gn < a.N) a.C[gm * a.ldc + gn] = make_double2(cre[i][j][e], cim[i][j][e]);
             }
+}
+
+// Every product that does not fill the chip with 64 x 128 tiles: an operator
+// on some modes of a state (M = K = the operator's dimension, N the rest of
+// the lattice), narrow or short products, batches.  A wave owns RT tiles of
+// 16 x 16 (every row of a tile row, 16 columns) and a workgroup four waves side
+// by side, so an element of B belongs to one wave: it goes from memory to the
+// operand registers without LDS and is read once per tile row.  Only A is
+// staged in LDS, in K chunks of BK (two buffers).  RT = ceil(M / 16) / tile
+// rows leaves at most 15 padded rows per tile row (M = 100: 112 rows).  The
+// products of a batch that share A are one product with `cols` = batch * N
+// columns (a lane finds its column's product), so only the last strip has
+// padded columns; otherwise cols = N and grid z is the product.  The sums and
+// their order are those of zgemm_mfma_kernel.
+// Bound by the matrix pipe for K = 100: 100 x 10^6 x 100 in 1584 us (50.5
+// TFLOP/s, 57 with the padded rows; 1855 us with 128 x 128 tiles), and by HBM
+// for K = 10: 10 x 10^7 x 10 in 623 us, 5.1 TB/s (1457 us with 64 x 128 tiles).
+// 10^4 products 100 x 100 x 100 with a shared A: 1579 us, 1985 with a grid z
+// entry each (128 computed columns for 100).
+// Measured slower at 100 x 10^6 x 100: two or eight waves a workgroup (1641, 1743),
+// chunks of 16 (1587) or 4 (1627), persistent workgroups that load their next
+// tile's first chunk early (1870).
+template <int RT, int BK>
+__global__ __launch_bounds__(256, 2) void zgemm_strip_kernel(ZgemmArgs a, int64_t cols) {
+    constexpr int BM = RT * 16, NT = 256, NW = 4;
+    a.A += int64_t(blockIdx.z) * a.sA;
+    __shared__ double sAr[2][BK][BM + 1], sAi[2][BK][BM + 1];
+    const int t = threadIdx.x;
+    const int lane = t & (MM_WAVE - 1), wave = t / MM_WAVE;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int64_t m0 = int64_t(blockIdx.y) * BM;
+    // this lane's column of B and C
+    const int64_t c = (int64_t(blockIdx.x) * NW + wave) * 16 + lr;
+    const bool col = c < cols;
+    const int64_t z = cols > a.N ? c / a.N : 0, n = c - z * a.N;
+    const double2 *const Bc = a.B + (z + blockIdx.z) * a.sB + n;
+    double2 *const Cc = a.C + (z + blockIdx.z) * a.sC + n;
+    const double2 zero = make_double2(0.0, 0.0);
+
+    dbl4 cre[RT], cim[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+        cre[i] = dbl4{0.0, 0.0, 0.0, 0.0};
+        cim[i] = dbl4{0.0, 0.0, 0.0, 0.0};
+    }
+    constexpr int NA = (BM * BK + NT - 1) / NT, NB = BK / 4;
+    double2 pa[NA], pb[NB];
+    auto load = [&](int64_t k0) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int e = t + i * NT;
+            const int r = e / BK, c = e % BK;
+            const int64_t gm = m0 + r, gk = k0 + c;
+            pa[i] = (r < BM && gm < a.M && gk < a.K) ? a.A[gm * a.lda + gk] : zero;
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int64_t gk = k0 + 4 * i + lk;
+            pb[i] = (col && gk < a.K) ? Bc[gk * a.ldb] : zero;
+        }
+    };
+    auto store_a = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int e = t + i * NT;
+            const int r = e / BK, c = e % BK;
+            if (r < BM) {
+                sAr[buf][c][r] = pa[i].x;
+                sAi[buf][c][r] = pa[i].y;
+            }
+        }
+    };
+    load(0);
+    store_a(0);
+    __syncthreads();
+    int buf = 0;
+    for (int64_t k0 = 0; k0 < a.K; k0 += BK) {
+        const bool more = k0 + BK < a.K;
+        double2 bk[NB];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) bk[i] = pb[i];
+        if (more) load(k0 + BK);
+#pragma unroll
+        for (int ks = 0; ks < NB; ++ks) {
+            if (ks && k0 + 4 * ks >= a.K) break;  // nothing but zeros past K
+            const double br = bk[ks].x, bi = bk[ks].y, nbi = -bi;
+            double ar[RT], ai[RT];
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                ar[i] = sAr[buf][4 * ks + lk][i * 16 + lr];
+                ai[i] = sAi[buf][4 * ks + lk][i * 16 + lr];
+            }
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                cre[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], br, cre[i], 0, 0, 0);
+                cim[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], bi, cim[i], 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                cre[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[i], nbi, cre[i], 0, 0, 0);
+                cim[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[i], br, cim[i], 0, 0, 0);
+            }
+        }
+        if (more) store_a(buf ^ 1);
+        __syncthreads();
+        buf ^= 1;
+    }
+    if (!col) return;
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t gm = m0 + i * 16 + lk + 4 * e;
+            if (gm < a.M) Cc[gm * a.ldc] = make_double2(cre[i][e], cim[i][e]);
+        }
 }
 
 }  // namespace mm
