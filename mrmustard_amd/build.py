@@ -17,6 +17,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 SOURCES = [
     "hermite.hip",
+    "stable.hip",
     "lds_3f.hip",
     "lds_3.hip",
     "lds_8f.hip",
