@@ -146,12 +146,23 @@ __device__ __forceinline__ Span xcd_span(int64_t blk, int64_t nblk, int64_t S) {
     return s;
 }
 
+// x / d for x * d < 2^32 by one multiplication: m = divide_magic(d).
+inline uint32_t divide_magic(uint32_t d) { return d == 1 ? 0u : uint32_t(((uint64_t(1) << 32) + d - 1) / d); }
+__device__ __forceinline__ int divide(int x, uint32_t m) { return m ? int(__umulhi(uint32_t(x), m)) : x; }
+
 // ------------------------------------------------------------ wave helpers
 
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Barrier for LDS traffic alone.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 __device__ __forceinline__ double shfl_xor_d(double v, int mask) {

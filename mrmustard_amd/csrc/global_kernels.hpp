@@ -122,25 +122,30 @@ __global__ __launch_bounds__(256) void fwd_slab_kernel(SlabArgs a) {
 }
 
 // --------------------------------------------- several slabs per launch
-// Slabs m0 .. m0 + T - 1 of level d in one launch (T = 1 or 2), for slabs
-// small enough that a launch per slab costs more than the slab's work: one
-// block per CU, 1024 threads, packed digits and an LDS coefficient table
-// (32-bit index arithmetic; fwd_slab_kernel takes any slab size).  A point
-// of slab m reads slab m - 1 at most h = stride[d+1] points back
-// (k - 1_d - 1_j, j > d) and slab m - 2 at itself, so block b, owning the
-// points [a_b, e_b) of every slab, computes slab m0 + s (phase s) on
-// [a_b - (T-1-s) h, e_b): its own points and those its later phases read.
-// A phase's values stay in LDS for the next phase (two buffers); a point's
-// own values of the two slabs below
-// stay in the registers of the thread that owns the point in every phase
-// (points are numbered from e_b down, so a region that shrinks from the
-// front keeps the numbering); phase 0 loads them and the point's neighbours
-// in slab m0 - 1 in one round trip.  Only owned points are written to G,
-// each by the expression of fwd_slab_kernel, so G is bit for bit the same;
-// a term with k_j = 0 is added as the reference adds it, a zero coefficient
+// Slabs m0 .. m0 + T - 1 of level d in one launch, for slabs small enough
+// that a launch per slab costs more than the slab's work: one block of 1024
+// threads per CU, packed digits and an LDS coefficient table (32-bit index
+// arithmetic; fwd_slab_kernel takes any slab size).  A point of slab m reads
+// slab m - 1 at its neighbours one below along the axes j > d and both slabs
+// below at itself, so a block that owns a box of the axes > d computes slab
+// m0 + s (phase s) on the box and on what its later phases read: the cells at
+// most T - 1 - s below it, summed over the axes.  The cells of that larger
+// box keep their place for the whole launch: a phase's values go through LDS
+// to the next phase (two buffers), and a cell's own values of the two slabs
+// below stay in the registers of its thread.  Phase 0 loads them and the
+// neighbours in slab m0 - 1.  Only owned points are written to G, each by
+// the expression of fwd_slab_kernel, so G is bit for bit the same; a term
+// with k_j = 0 is added as the reference adds it, a zero coefficient
 // A_dj sqrt(0) times a value read at the point itself (no branch per lane).
+// A box has few cells below it where a run of consecutive points of the same
+// size has the whole of its outer neighbours: of the (40,)^4 density matrix
+// (39 slabs of 64,000 points) a block of 250 consecutive points computes 1,850
+// for two slabs.  Measured there, the whole forward: 193 ->
+// 148 us (four slabs a launch, boxes of 4 x 8 x 8 points); (60,)^3 161 -> 83 us,
+// (300, 80, 60) 678 -> 279 us, (500, 150, 20) 1118 -> 474 us.
 constexpr int MULTI_THREADS = 1024;
-constexpr int MULTI_KMAX = 2;  // points per thread: regions of at most 2048 points
+constexpr int MULTI_KMAX = 2;  // cells per thread (KM): more measured slower than a launch per slab
+constexpr int MULTI_CELLS = MULTI_THREADS * MULTI_KMAX;
 
 struct SlabMultiArgs {
     Geom g;
@@ -149,54 +154,75 @@ struct SlabMultiArgs {
     const double *sq, *rsq;
     int *nf;  // raised when a stored value is not finite
     int d, m0, nphase;
-    int tile, halo, cap;    // owned points per block, neighbour reach, points per LDS buffer
+    int e[8], nt[8], h[8], ls[8];  // axes > d: points of a box, boxes, cells below it (0 where the box spans the axis), cell strides
+    uint32_t lsm[8];        // divide_magic of ls
+    int cells;
     int smax;               // row length of the coefficient table (largest shape of the axes > d)
     int kbit[8], kmask[8];  // packed digits of the axes > d
 };
 
-template <int D>
+template <int D, int KM>
 __global__ __launch_bounds__(MULTI_THREADS) void fwd_slab_multi_kernel(SlabMultiArgs a) {
     extern __shared__ __align__(16) char lds[];
     double2 *buf0 = reinterpret_cast<double2 *>(lds);
-    double2 *buf1 = buf0 + a.cap;
-    double2 *ctab = buf1 + a.cap;  // A_dj sqrt(k_j) for j > d, row j - d - 1
+    double2 *buf1 = buf0 + (a.nphase > 1 ? a.cells : 0);
+    double2 *ctab = buf1 + (a.nphase > 2 ? a.cells : 0);  // A_dj sqrt(k_j) for j > d, row j - d - 1
     const double2 zero = make_double2(0.0, 0.0);
-    const int d = a.d, T = a.nphase, h = a.halo;
+    const int d = a.d, T = a.nphase;
     const int Sd = int(a.g.stride[d]);
     for (int t = threadIdx.x; t < (D - 1 - d) * a.smax; t += blockDim.x) {
         const int j = d + 1 + t / a.smax, k = t % a.smax;
         ctab[t] = k < a.g.shape[j] ? cscale_promoted(a.A[d * D + j], a.sq[k]) : zero;
     }
-    const int ab = int(xcd_block(blockIdx.x, gridDim.x)) * a.tile;
-    const int eb = min(ab + a.tile, Sd);
-    const int lo0 = max(0, ab - (T - 1) * h);
-    int st[D];
+    int st[D], base[D];
+    {
+        int r = int(xcd_block(blockIdx.x, gridDim.x));
 #pragma unroll
-    for (int j = 0; j < D; ++j) st[j] = int(a.g.stride[j]);
-    uint32_t kp[MULTI_KMAX];
-    double2 p1v[MULTI_KMAX], p2v[MULTI_KMAX], nb[MULTI_KMAX][D];
+        for (int j = D - 1; j >= 0; --j) {
+            st[j] = int(a.g.stride[j]);
+            base[j] = 0;
+            if (j <= d) continue;
+            const int tj = r % a.nt[j];
+            r /= a.nt[j];
+            base[j] = tj * a.e[j];
+        }
+    }
+    // cell x0 + r * 1024 of this thread: its point of a slab, the cells it
+    // lies below the box (T: no point), its packed digits
+    uint32_t kp[KM];
+    int qv[KM], under[KM];
+    double2 p1v[KM], p2v[KM], nb0[KM][D];
     const int64_t base0 = int64_t(a.m0) * Sd;
     const double2 *G0 = a.G + base0 - Sd;  // slab m0 - 1
 #pragma unroll
-    for (int r = 0; r < MULTI_KMAX; ++r) {
-        const int q = eb - 1 - int(threadIdx.x) - r * MULTI_THREADS;
+    for (int r = 0; r < KM; ++r) {
+        const int x = int(threadIdx.x) + r * int(blockDim.x);
+        int rem = x, u = 0, q = 0;
+        bool in = x < a.cells;
         kp[r] = 0;
+#pragma unroll
+        for (int j = 0; j < D; ++j) {
+            if (j <= d) continue;
+            const int cj = divide(rem, a.lsm[j]);
+            rem -= cj * a.ls[j];
+            const int kj = base[j] + cj - a.h[j];
+            u += max(0, a.h[j] - cj);
+            in = in && kj >= 0 && kj < a.g.shape[j] && cj < a.e[j] + a.h[j];
+            q += kj * st[j];
+            kp[r] |= uint32_t(max(kj, 0)) << a.kbit[j];
+        }
+        under[r] = in ? u : T;
+        qv[r] = in ? q : 0;
         p1v[r] = zero;
         p2v[r] = zero;
-#pragma unroll
-        for (int j = 0; j < D; ++j) nb[r][j] = zero;
-        if (q >= lo0) {
-            int rem = q;
-#pragma unroll
-            for (int j = 0; j < D; ++j) {
-                if (j <= d) continue;
-                const int kj = rem / st[j];
-                rem -= kj * st[j];
-                kp[r] |= uint32_t(kj) << a.kbit[j];
-                nb[r][j] = G0[kj > 0 ? q - st[j] : q];  // phase 0's neighbours, loaded with the point's own values
-            }
+        if (under[r] < T) {
             p1v[r] = G0[q];
             if (a.m0 >= 2) p2v[r] = G0[q - Sd];
+#pragma unroll
+            for (int j = 1; j < D; ++j) {
+                if (j <= d) continue;
+                nb0[r][j] = G0[((kp[r] >> a.kbit[j]) & uint32_t(a.kmask[j])) ? q - st[j] : q];
+            }
         }
     }
     __syncthreads();  // the coefficient table
@@ -204,36 +230,40 @@ __global__ __launch_bounds__(MULTI_THREADS) void fwd_slab_multi_kernel(SlabMulti
     bool bad = false;
     for (int s = 0; s < T; ++s) {
         const int m = a.m0 + s;
-        const int lo = max(0, ab - (T - 1 - s) * h);
-        const int plo = max(0, ab - (T - s) * h);  // origin of the previous phase's buffer
         const double2 *prev = (s & 1) ? buf0 : buf1;
         double2 *cur = (s & 1) ? buf1 : buf0;
         const double2 cdd = cscale_promoted(a.A[d * D + d], a.sq[m > 0 ? m - 1 : 0]);
         const double sm = a.sq[m], rm = a.rsq[m];
 #pragma unroll
-        for (int r = 0; r < MULTI_KMAX; ++r) {
-            const int q = eb - 1 - int(threadIdx.x) - r * MULTI_THREADS;
-            if (q < lo) continue;
+        for (int r = 0; r < KM; ++r) {
+            if (under[r] >= T - s) continue;
+            const int x = int(threadIdx.x) + r * int(blockDim.x), q = qv[r];
+            // k_j = 0: the point itself times the zero coefficient A_dj sqrt(0)
+            double2 nb[D];
+            int kj[D];
+#pragma unroll
+            for (int j = 1; j < D; ++j) {
+                if (j <= d) continue;
+                kj[j] = int((kp[r] >> a.kbit[j]) & uint32_t(a.kmask[j]));
+                nb[j] = s == 0 ? nb0[r][j] : prev[kj[j] > 0 ? x - a.ls[j] : x];
+            }
             double2 v = cmul(bd, p1v[r]);
             if (m >= 2) v = cadd(v, cmul(cdd, p2v[r]));
 #pragma unroll
             for (int j = 1; j < D; ++j) {
                 if (j <= d) continue;
-                const int kj = int((kp[r] >> a.kbit[j]) & uint32_t(a.kmask[j]));
-                // k_j = 0: the point itself times the zero coefficient A_dj sqrt(0)
-                const double2 nbv = s == 0 ? nb[r][j] : prev[(kj > 0 ? q - st[j] : q) - plo];
-                v = cadd(v, cmul(ctab[(j - d - 1) * a.smax + kj], nbv));
+                v = cadd(v, cmul(ctab[(j - d - 1) * a.smax + kj[j]], nb[j]));
             }
             const double2 out = cdiv_by(v, sm, rm);
-            if (s + 1 < T) cur[q - lo] = out;
-            if (q >= ab) {
+            if (s + 1 < T) cur[x] = out;
+            if (under[r] == 0) {
                 a.G[int64_t(m) * Sd + q] = out;
                 bad = bad || !finite2(out);
             }
             p2v[r] = p1v[r];
             p1v[r] = out;
         }
-        __syncthreads();
+        lds_barrier();  // stores to G need no wait: no later phase reads them
     }
     if (__builtin_expect(bad, 0) && a.nf) atomicOr(a.nf, 1);
 }

@@ -373,47 +373,99 @@ int launch_slab(const SlabArgs &a, int D, int64_t Sd, int num_cu, hipStream_t s)
     return MM_OK;
 }
 
-// Slabs of level d of at most 2^17 points, whose launch costs more than
-// their work, go through fwd_slab_multi_kernel: the slab cut into one tile
-// per CU, two slabs per launch when a block's first region (tile + halo)
-// stays within 2048 points and two region buffers within the LDS, else one.
-// Measured on the (40,)^4 density matrix (39 level-0 slabs of 64,000 points),
-// the whole forward: one slab per launch of fwd_slab_kernel 246 us, of this
-// kernel 219 us, two per launch 199 us; three per launch measured no faster
-// than two (a block's redundant halo points cost about as much as the
-// launches they save).
+// Slabs of level d of at most 2^18 points go through fwd_slab_multi_kernel
+// where that is estimated to be quicker: boxes of at most one per CU, T slabs
+// a launch.  For each T the axis whose next cut saves the most cells for the
+// boxes it adds is cut until the boxes would outnumber the CUs.
 struct MultiPlan {
-    int nphase = 0, tile = 0, cap = 0, nblk = 0, smax = 1;
+    int nphase = 0, cells = 0, nblk = 0, smax = 1;
+    int e[8], nt[8], h[8];
     int64_t shmem = 0;
+    double us = 0.0;  // estimated time of a slab
 };
 
-bool multi_plan(const Shape &S, int d, const DevState *ds, MultiPlan *p) {
-    if (d + 1 >= S.D || S.s[d] < 2) return false;
+// One slab in a launch of its own (fwd_slab_kernel): measured 6.9 us at 248,832
+// points of D = 6, 22.7 at 10^6 of D = 8.
+double slab_us(int64_t Sd) { return std::max(4.5, 2.0 + double(Sd) / 50e3); }
+
+bool multi_plan(const Shape &S, int d, const DevState *ds, MultiPlan *best) {
+    const int D = S.D;
+    if (d + 1 >= D || S.s[d] < 2) return false;
     const int64_t Sd = S.st[d];
-    if (Sd > (int64_t(1) << 17)) return false;
-    const int64_t h = S.st[d + 1];
+    if (Sd > (int64_t(1) << 18)) return false;
     int bits = 0, smax = 1;
-    for (int j = d + 1; j < S.D; ++j) {
+    for (int j = d + 1; j < D; ++j) {
         int w = 0;
         while ((1 << w) < S.s[j]) ++w;
         bits += w;
         smax = std::max(smax, int(S.s[j]));
     }
     if (bits > 32) return false;
-    const int64_t tile = std::max<int64_t>(64, (Sd + ds->num_cu - 1) / ds->num_cu);
-    for (int T = 2; T >= 1; --T) {
-        const int64_t cap = std::min<int64_t>(Sd, tile + (T - 1) * h);
-        const int64_t shmem = 2 * cap * 16 + int64_t(S.D - 1 - d) * smax * 16;
-        if (cap > int64_t(MULTI_THREADS) * MULTI_KMAX || shmem > ds->max_lds) continue;
-        p->nphase = T;
-        p->tile = int(tile);
-        p->cap = int(cap);
-        p->nblk = int((Sd + tile - 1) / tile);
-        p->smax = smax;
-        p->shmem = shmem;
-        return true;
+    const int64_t tab = int64_t(D - 1 - d) * smax * 16;
+    bool found = false;
+    for (int T : {1, 2, 3, 4, 6, 8, 12}) {
+        if (T > S.s[d] - 1 && T > 1) break;
+        MultiPlan p;
+        p.nphase = T;
+        p.smax = smax;
+        int64_t blocks = 1;
+        for (int j = d + 1; j < D; ++j) {
+            p.nt[j] = 1;
+            p.e[j] = S.s[j];
+            p.h[j] = 0;
+        }
+        for (;;) {
+            double cells = 1.0, own = 1.0;
+            for (int j = d + 1; j < D; ++j) {
+                cells *= p.e[j] + p.h[j];
+                own *= p.e[j];
+            }
+            p.cells = int(std::min(cells, 1e9));
+            p.nblk = int(blocks);
+            p.shmem = (T > 2 ? 2 : T - 1) * int64_t(p.cells) * 16 + tab;
+            if (p.cells <= MULTI_CELLS && p.shmem <= ds->max_lds) {
+                // 4.2 us a launch (5.7 with two cells a thread), 0.27 us a wave
+                // on each SIMD and phase, the later phases on ever fewer cells
+                double us = cells > MULTI_THREADS ? 5.7 : 4.2;
+                for (int s = 0; s < T; ++s) {
+                    const double here = T > 1 ? own + (cells - own) * double(T - 1 - s) / double(T - 1) : own;
+                    us += 0.3 + 0.27 * std::ceil(here / 256.0);
+                }
+                const double groups = double((S.s[d] - 1 + T - 1) / T);
+                p.us = us * groups / double(S.s[d] - 1);
+                if (!found || p.us < best->us) *best = p;
+                found = true;
+            }
+            // the cut that saves most
+            int jb = -1, eb = 0, nb = 0;
+            double gain = 0.0;
+            for (int j = d + 1; j < D; ++j) {
+                if (p.e[j] <= 1) continue;
+                const int n = (S.s[j] + p.e[j] - 2) / (p.e[j] - 1), e = (S.s[j] + n - 1) / n;
+                if (blocks / p.nt[j] * n > ds->num_cu) continue;
+                // (one slab a launch: runs of consecutive points, the outer axes first)
+                const double save = T == 1 ? 0.0 : std::log(double(p.e[j] + p.h[j]) / double(e + T - 1)) / std::log(double(n) / p.nt[j]);
+                if (jb < 0 || save > gain) {
+                    gain = save;
+                    jb = j;
+                    eb = e;
+                    nb = n;
+                }
+            }
+            if (jb < 0) break;
+            blocks = blocks / p.nt[jb] * nb;
+            p.nt[jb] = nb;
+            p.e[jb] = eb;
+            p.h[jb] = T - 1;
+        }
     }
-    return false;
+    return found && best->us < slab_us(Sd);
+}
+
+template <int D, int KM>
+void launch_multi_t(const SlabMultiArgs &a, const MultiPlan &p, int threads, hipStream_t s) {
+    raise_lds_limit(fwd_slab_multi_kernel<D, KM>, int(p.shmem));
+    hipLaunchKernelGGL((fwd_slab_multi_kernel<D, KM>), dim3(unsigned(p.nblk)), dim3(unsigned(threads)), size_t(p.shmem), s, a);
 }
 
 int launch_slab_multi(const SlabArgs &sa, const Shape &S, const MultiPlan &p, int d, int m0, int T, hipStream_t s) {
@@ -429,24 +481,28 @@ int launch_slab_multi(const SlabArgs &sa, const Shape &S, const MultiPlan &p, in
     a.d = d;
     a.m0 = m0;
     a.nphase = T;
-    a.tile = p.tile;
-    a.halo = int(S.st[d + 1]);
-    a.cap = p.cap;
+    a.cells = p.cells;
     a.smax = p.smax;
-    int bit = 0;
+    int bit = 0, ls = 1;
     for (int j = S.D - 1; j > d; --j) {
+        a.e[j] = p.e[j];
+        a.nt[j] = p.nt[j];
+        a.h[j] = p.h[j];
+        a.ls[j] = ls;
+        a.lsm[j] = divide_magic(uint32_t(ls));
+        ls *= p.e[j] + p.h[j];
         int w = 0;
         while ((1 << w) < S.s[j]) ++w;
         a.kbit[j] = bit;
         a.kmask[j] = (1 << w) - 1;
         bit += w;
     }
-    const dim3 grid(unsigned(p.nblk)), block(MULTI_THREADS);
+    const int km = p.cells <= MULTI_THREADS ? 1 : MULTI_KMAX;
+    const int threads = ((p.cells + km - 1) / km + MM_WAVE - 1) / MM_WAVE * MM_WAVE;
     switch (S.D) {
-#define CASE(DD)                                                                                      \
-    case DD:                                                                                          \
-        raise_lds_limit(fwd_slab_multi_kernel<DD>, int(p.shmem));                                     \
-        hipLaunchKernelGGL((fwd_slab_multi_kernel<DD>), grid, block, size_t(p.shmem), s, a);          \
+#define CASE(DD)                                                                                              \
+    case DD:                                                                                                  \
+        km == 1 ? launch_multi_t<DD, 1>(a, p, threads, s) : launch_multi_t<DD, MULTI_KMAX>(a, p, threads, s); \
         break;
         CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
@@ -475,6 +531,28 @@ int launch_level(SlabArgs sa, const Shape &S, int d, const DevState *ds, hipStre
         if (rc) return rc;
     }
     return MM_OK;
+}
+
+// Largest slab of a sub-lattice of Ds indices that one workgroup steps through
+// quicker than launches over all CUs do (a launch of fwd_slab_multi_kernel
+// costs 0.7 to 1.5 us a slab).  Measured at both, the whole forward: with
+// three indices left, 900-point slabs ((30,)^4) 88 against 95 us, 1,089 equal,
+// 1,600 ((40,)^3) 70 against 64, 2,744 ((14,)^5) 119 against 80, 3,600 ((60,)^4)
+// 440 against 294; with more, 729 ((9,)^7) 185 against 178, 1,728 ((12,)^6) 151
+// against 130, 4,096 ((8,)^6) 96 against 62.
+int64_t face_points(int Ds) { return Ds <= 3 ? 1500 : 700; }
+
+// The level from which one workgroup sweeps a larger lattice's face, no lower
+// than `top` (which fits); *T its threads.
+int face_top(const Shape &S, int top, const DevState *ds, int *T) {
+    MultiPlan p;
+    while (top + 2 < S.D && S.st[top] > face_points(S.D - top) && multi_plan(S, top, ds, &p)) {
+        const int Tn = team_threads(S.st[top + 1], lds_maxt(S.D, false));
+        if (lds_bytes(S, top + 1, false, Tn / MM_WAVE, kernel_dmax(S.D)) > ds->max_lds || !packed_bits_ok(S, top + 1)) break;
+        ++top;
+        *T = Tn;
+    }
+    return top;
 }
 
 // ------------------------------------------------------ non-finite fix-up
@@ -787,13 +865,12 @@ int launch_stable(const Shape &S, int64_t B, const double *A, const double *b, c
 
 // Workspace of one vanilla forward (+ fused VJP when `fused`).
 // A single triple (D >= 3) whose level-0 slab fits in LDS but holds more
-// than 3072 points (four or more per thread of the workgroup; with the VJP,
-// more than 1024) is swept over all CUs: the face {k_0 = 0} in LDS (team size
-// *Tf), then the level-0 slabs.  Measured for the forward: a workgroup step
-// costs ~1.7 us at three points per thread and ~3.4 us at four, a slab over
-// all CUs ~2.3 us (two per launch); a fused workgroup step adds the VJP terms.
+// points than FACE_POINTS (with the VJP, more than 1024) is swept over all CUs:
+// the face {k_0 = 0} in LDS (team size *Tf), then the level-0 slabs.  Measured
+// for the forward: (100, 50, 50) 189 -> 113 us, (40,)^3 70 -> 64 us, but
+// (30, 35, 40) 48 -> 51 us; a fused workgroup step adds the VJP terms.
 bool spread_single(const Shape &S, bool fused, int64_t B, const DevState *ds, int *Tf) {
-    if (B != 1 || S.D < 3 || S.st[0] <= (fused ? 1024 : 3072) || !packed_bits_ok(S, 1)) return false;
+    if (B != 1 || S.D < 3 || S.st[0] <= (fused ? 1024 : face_points(S.D)) || !packed_bits_ok(S, 1)) return false;
     int T = 64;
     if (choose_top(S, fused, ds->max_lds, lds_maxt(S.D, fused), &T) != 0) return false;
     *Tf = team_threads(S.st[1], lds_maxt(S.D, false));
@@ -848,10 +925,11 @@ int vanilla_uniform(const Shape &S, int64_t B, const double *A, const double *b,
     // Large lattice: LDS sweep of the sub-lattice {k_<top = 0}, then one launch
     // per slab for the levels above, then the VJP reduction.
     if (spread) {
-        top = 1;
         T = Tf;
+        top = face_top(S, 1, ds, &T);
     } else {
         top = choose_top(S, false, ds->max_lds, lds_maxt(S.D, false), &T);
+        top = face_top(S, top, ds, &T);
     }
     if (fused && (!ws || ws_bytes < vjp_min_ws_bytes(S, B)))
         return fail(MM_ERR_WORKSPACE, "fused workspace of %zu bytes needed, %zu given", vjp_ws_bytes(S, B), ws_bytes);
@@ -950,6 +1028,7 @@ int window_face(const Shape &S, const double *A, const double *b, const double *
         if (lds_bytes(S, 1, false, T / MM_WAVE, kernel_dmax(S.D)) > ds->max_lds || !packed_bits_ok(S, 1))
             return fail(MM_ERR_UNSUPPORTED, "slab window: face does not fit in LDS");
     }
+    top = face_top(S, top, ds, &T);
     LdsArgs a;
     memset(&a, 0, sizeof(a));
     a.P = bases(A, b, c, nullptr, reinterpret_cast<double *>(face), nullptr, nullptr, nullptr, nullptr);

@@ -61,19 +61,8 @@ struct StableTileArgs {
     uint16_t order[STABLE_TILE_ROWS];  // the rows of a tile by digit sum
 };
 
-// x / d for x * d < 2^32 by one multiplication: m = divide_magic(d).
-inline uint32_t divide_magic(uint32_t d) { return d == 1 ? 0u : uint32_t(((uint64_t(1) << 32) + d - 1) / d); }
-__device__ __forceinline__ int divide(int x, uint32_t m) { return m ? int(__umulhi(uint32_t(x), m)) : x; }
-
 // Lanes per point.
 constexpr int stable_lanes(int D) { return D <= 2 ? 2 : (D <= 4 ? 4 : 8); }
-
-// Barrier for LDS traffic alone.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 // DPP move of a complex value; every lane that is read is active.
 template <int CTRL>
