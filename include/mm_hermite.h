@@ -241,6 +241,14 @@ int mm_hermite_1leftover_vjp(const double *A, const double *b, const double *c, 
                              int Mt, int reordered, const double *dLdout, double *out, double *dA, double *db, double *dc,
                              void *workspace, size_t ws_bytes, void *stream);
 
+/* The same reverse sweep from the workspace that mm_hermite_1leftover filled
+ * for the same triple and cutoffs (fwd_ws, only read), in torch's convention:
+ * for grad = dL/d(conj out), conj(VJP(conj(grad))).  No forward is run. */
+size_t mm_hermite_1leftover_grad_workspace(int64_t output_cutoff, const int64_t *pnr_cutoffs, int Mt);
+int mm_hermite_1leftover_grad(const double *A, const double *b, const double *c, int64_t output_cutoff, const int64_t *pnr_cutoffs,
+                              int Mt, int reordered, const void *fwd_ws, size_t fwd_bytes, const double *grad, double *dA, double *db,
+                              double *dc, void *workspace, size_t ws_bytes, void *stream);
+
 /* The Fock array of a triple with derived variables, the lattice never
  * stored whole: out[h] = sum_k G[h, k] w[k], G the lattice of (A, b, c) on
  * `shape` (D axes), h its first n_head axes, k the other D - n_head axes

@@ -173,7 +173,7 @@ void launch_diag_vjp(DiagVjpArgs &v, const std::vector<int64_t> &counts, int nbl
         const int iters = int((counts[w] + per - 1) / per);
         hipLaunchKernelGGL((diag_vjp_kernel<M, REORDER>), dim3(nw), dim3(DG_THREADS), 0, s, v, w, counts[w], starts[w], iters);
     }
-    hipLaunchKernelGGL((diag_vjp_finalize<M, REORDER>), dim3(2 * M * (2 * M + 1)), dim3(256), 0, s, v.part, nblk, dA, dB);
+    hipLaunchKernelGGL((diag_vjp_finalize<M, REORDER>), dim3(2 * M * (2 * M + 1)), dim3(256), 0, s, v.part, nblk, dA, dB, 1.0);
 }
 
 // ------------------------------------------------------------ one leftover mode
@@ -311,7 +311,35 @@ void launch_lo_vjp(LeftVjpArgs &v, const std::vector<int64_t> &counts, int nblk,
     int nt = 64;
     while (nt < v.a.c0) nt <<= 1;  // c0 <= 1024
     hipLaunchKernelGGL((lo_init_vjp_kernel<MT, REORDER>), dim3(1), dim3(nt), 0, s, v, nblk);
-    hipLaunchKernelGGL((diag_vjp_finalize<MT + 1, REORDER>), dim3(GL * (GL + 1)), dim3(256), 0, s, v.part, nblk + 1, dA, dB);
+    hipLaunchKernelGGL((diag_vjp_finalize<MT + 1, REORDER>), dim3(GL * (GL + 1)), dim3(256), 0, s, v.part, nblk + 1, dA, dB, v.gsign);
+}
+
+// The reverse sweep with its arrays in ws (lo_vjp_bytes without the forward's).
+int lo_reverse(LeftVjpArgs &v, const DiagGeom &g, int Mt, int reordered, const double *cot, double *dA, double *db, double *dc, char *ws,
+               int nblk, const std::vector<int64_t> &counts, hipStream_t s) {
+    const int64_t P = g.a.P, C = v.a.C;
+    const int64_t nmirror = C * (4 * Mt * P + g.n2 + 2 * g.n11);
+    v.cot = reinterpret_cast<const double2 *>(cot);
+    v.adD = reinterpret_cast<double2 *>(ws);
+    v.adO = v.adD + 2 * Mt * P * C;
+    v.ad2 = v.adO + 2 * Mt * P * C;
+    v.ad1010 = v.ad2 + g.n2 * C;
+    v.ad1001 = v.ad1010 + g.n11 * C;
+    v.adP = reinterpret_cast<double2 *>(ws + align256(size_t(16) * size_t(nmirror)));
+    v.part = reinterpret_cast<double2 *>(reinterpret_cast<char *>(v.adP) + align256(size_t(16) * size_t(Mt * P * C)));
+    v.dc = reinterpret_cast<double2 *>(dc);
+    double2 *dA2 = reinterpret_cast<double2 *>(dA), *dB2 = reinterpret_cast<double2 *>(db);
+    switch (Mt * 2 + (reordered ? 1 : 0)) {
+#define CASE(MM)                                                                \
+    case 2 * MM: launch_lo_vjp<MM, false>(v, counts, nblk, dA2, dB2, s); break; \
+    case 2 * MM + 1: launch_lo_vjp<MM, true>(v, counts, nblk, dA2, dB2, s); break;
+        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
+#undef CASE
+        default:
+            return fail(MM_ERR_INVALID, "bad number of detected modes");
+    }
+    LAUNCH_CHECK("lo vjp kernels");
+    return MM_OK;
 }
 
 }  // namespace
@@ -375,29 +403,43 @@ int mm_hermite_1leftover_vjp(const double *A, const double *b, const double *c, 
     std::vector<int64_t> counts;
     rc = lo_forward(v.a, Mt, reordered, ds, s, &counts);
     if (rc) return rc;
-    const int64_t P = g.a.P;
-    const int64_t nmirror = C * (4 * Mt * P + g.n2 + 2 * g.n11);
-    v.cot = reinterpret_cast<const double2 *>(dLdout);
-    v.adD = reinterpret_cast<double2 *>(ws + align256(fwd_bytes));
-    v.adO = v.adD + 2 * Mt * P * C;
-    v.ad2 = v.adO + 2 * Mt * P * C;
-    v.ad1010 = v.ad2 + g.n2 * C;
-    v.ad1001 = v.ad1010 + g.n11 * C;
-    v.adP = reinterpret_cast<double2 *>(ws + align256(fwd_bytes) + align256(size_t(16) * size_t(nmirror)));
-    v.part = reinterpret_cast<double2 *>(reinterpret_cast<char *>(v.adP) + align256(size_t(16) * size_t(Mt * P * C)));
-    v.dc = reinterpret_cast<double2 *>(dc);
-    double2 *dA2 = reinterpret_cast<double2 *>(dA), *dB2 = reinterpret_cast<double2 *>(db);
-    switch (Mt * 2 + (reordered ? 1 : 0)) {
-#define CASE(MM)                                                                        \
-    case 2 * MM: launch_lo_vjp<MM, false>(v, counts, nblk, dA2, dB2, s); break; \
-    case 2 * MM + 1: launch_lo_vjp<MM, true>(v, counts, nblk, dA2, dB2, s); break;
-        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
-#undef CASE
-        default:
-            return fail(MM_ERR_INVALID, "bad number of detected modes");
-    }
-    LAUNCH_CHECK("lo vjp kernels");
-    return MM_OK;
+    v.gsign = 1.0;
+    return lo_reverse(v, g, Mt, reordered, dLdout, dA, db, dc, ws + align256(fwd_bytes), nblk, counts, s);
+}
+
+size_t mm_hermite_1leftover_grad_workspace(int64_t output_cutoff, const int64_t *pnr_cutoffs, int Mt) {
+    DiagGeom g;
+    int c0 = 0;
+    size_t bytes = 0;
+    if (lo_geom(output_cutoff, pnr_cutoffs, Mt, &g, &c0, &bytes)) return 0;
+    return lo_vjp_bytes(g, Mt, int64_t(c0) * c0, bytes, lo_vjp_blocks(g, Mt, int64_t(c0) * c0)) - align256(bytes);
+}
+
+int mm_hermite_1leftover_grad(const double *A, const double *b, const double *c, int64_t output_cutoff, const int64_t *pnr_cutoffs,
+                              int Mt, int reordered, const void *fwd_ws, size_t fwd_bytes, const double *grad, double *dA, double *db,
+                              double *dc, void *workspace, size_t ws_bytes, void *stream) {
+    DiagGeom g;
+    int c0 = 0;
+    size_t fwd_need = 0;
+    int rc = lo_geom(output_cutoff, pnr_cutoffs, Mt, &g, &c0, &fwd_need);
+    if (rc) return rc;
+    if (!A || !b || !c || !grad || !dA || !db || !dc) return fail(MM_ERR_INVALID, "NULL array pointer");
+    const int64_t C = int64_t(c0) * c0;
+    const int nblk = lo_vjp_blocks(g, Mt, C);
+    const size_t need = lo_vjp_bytes(g, Mt, C, fwd_need, nblk) - align256(fwd_need);
+    if (!fwd_ws || fwd_bytes < fwd_need)
+        return fail(MM_ERR_WORKSPACE, "1leftover workspace of %zu bytes expected, %zu given", fwd_need, fwd_bytes);
+    if (!workspace || ws_bytes < need)
+        return fail(MM_ERR_WORKSPACE, "1leftover gradient workspace of %zu bytes needed, %zu given", need, ws_bytes);
+    DevState *ds = nullptr;
+    rc = device_state(&ds);
+    if (rc) return rc;
+    LeftVjpArgs v;
+    // the reverse sweep only reads the forward's arrays, and no entry of out
+    lo_bind(g, c0, A, b, c, nullptr, static_cast<char *>(const_cast<void *>(fwd_ws)), ds, v.a);
+    v.gsign = -1.0;
+    return lo_reverse(v, g, Mt, reordered, grad, dA, db, dc, static_cast<char *>(workspace), nblk, diag_weight_counts(v.a.t, Mt),
+                      reinterpret_cast<hipStream_t>(stream));
 }
 
 size_t mm_hermite_diagonal_workspace(const int64_t *cutoffs, int M, int64_t nb) {

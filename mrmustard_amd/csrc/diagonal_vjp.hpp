@@ -276,9 +276,10 @@ __global__ __launch_bounds__(DG_THREADS) void diag_vjp_kernel(DiagVjpArgs v, int
 }
 
 // dA (caller's order), dB: one block per entry; thread k sums partial rows
-// k, k + 256, ... in order, then a fixed tree over the 256 threads.
+// k, k + 256, ... in order, then a fixed tree over the 256 threads.  gsign = -1:
+// written conjugated.
 template <int M, bool REORDER>
-__global__ __launch_bounds__(256) void diag_vjp_finalize(const double2 *part, int nblk, double2 *dA, double2 *dB) {
+__global__ __launch_bounds__(256) void diag_vjp_finalize(const double2 *part, int nblk, double2 *dA, double2 *dB, double gsign) {
     constexpr int G = 2 * M;
     __shared__ double2 red[256];
     const int e = blockIdx.x, k = threadIdx.x;
@@ -292,10 +293,11 @@ __global__ __launch_bounds__(256) void diag_vjp_finalize(const double2 *part, in
     }
     if (k == 0) {
         const int r = e / (G + 1), l = e % (G + 1);
+        const double2 sum = make_double2(red[0].x, gsign * red[0].y);
         if (l < G)
-            dA[src_index<M, REORDER>(r) * G + src_index<M, REORDER>(l)] = red[0];
+            dA[src_index<M, REORDER>(r) * G + src_index<M, REORDER>(l)] = sum;
         else
-            dB[src_index<M, REORDER>(r)] = red[0];
+            dB[src_index<M, REORDER>(r)] = sum;
     }
 }
 

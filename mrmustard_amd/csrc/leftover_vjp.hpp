@@ -38,20 +38,32 @@ struct LeftVjpArgs {
     double2 *adP;                     // adjoints of the arr1[2d, p] blocks from the off-diagonal pivots
     double2 *part;                    // (nblk + 1) x 2L x (2L + 1): dA rows, then dB
     double2 *dc;                      // adjoint of c
+    double gsign;                     // -1: the cotangent is read, dc written conjugated
 };
 
-// Output adjoints of the lane's block entry and of the entries (m+1, n),
-// (m, n+1) of the array at src (block entry innermost), divided by K.
-__device__ __forceinline__ void lo_out_adjoints(const double2 *src, const double2 *ext, int pos, int c0, bool up_m, bool up_n,
-                                                double K, double rK, double2 &wo, double2 &wm, double2 &wn) {
-    auto ob = [&](int e) {
-        double2 o = src[e];
-        if (ext) o = cadd(o, ext[e]);
-        return cdiv_by(o, K, rK);
-    };
-    wo = ob(pos);
-    if (up_m) wm = ob(pos + c0);
-    if (up_n) wn = ob(pos + 1);
+// One pivot's inputs of a lane, as loaded: the input its column carries, the
+// adjoints of its output at its own block entry and at (m+1, n), (m, n+1),
+// the pivot block's own and two lowered entries, and the roots that go with
+// them.  All loads are issued before the first use: what a launch of these
+// kernels costs is the round trips one after another, not its bytes (at two
+// detected modes, 400-entry blocks: off-diagonal 8.9 -> 7.1 us, diagonal 6.9 ->
+// 5.8 us a launch against loads where they are used and sums in LDS).
+struct LoIn {
+    double2 x, o, om, on, pv, pvm, pvn;
+    double sx, K, rK;
+};
+
+__device__ __forceinline__ void lo_clear(LoIn &q) {
+    q.x = q.o = q.om = q.on = q.pv = q.pvm = q.pvn = make_double2(0.0, 0.0);
+    q.sx = 0.0;
+    q.K = q.rK = 1.0;
+}
+
+// Output adjoints at src (block entry innermost).
+__device__ __forceinline__ void lo_load_adjoints(const double2 *src, int pos, int c0, bool up_m, bool up_n, LoIn &q) {
+    q.o = src[pos];
+    if (up_m) q.om = src[pos + c0];
+    if (up_n) q.on = src[pos + 1];
 }
 
 // Lane (i, slot) of output row r = i + 2: its term of the pivot-block adjoint.
@@ -65,11 +77,14 @@ __device__ __forceinline__ double2 lo_piv_term(const double2 (*sA)[2 * L], const
 }
 
 // Per-block sums over the PB params slots of each pivot row (rows 2 ..), added
-// to this block's partial row.
+// to this block's partial row: lane t's dA row (l < GL) and dB (l == GL) in acc.
 template <int MT>
-__device__ __forceinline__ void lo_vjp_flush(double2 *part, const double2 (*sacc)[DG_THREADS]) {
+__device__ __forceinline__ void lo_vjp_flush(double2 *part, const double2 (&acc)[2 * MT + 3], double2 (*sacc)[DG_THREADS]) {
     constexpr int G = 2 * MT, GL = G + 2;
     constexpr int PB = DG_THREADS / G;
+#pragma unroll
+    for (int l = 0; l <= GL; ++l) sacc[l][threadIdx.x] = acc[l];
+    __syncthreads();
     double2 *prow = part + int64_t(blockIdx.x) * GL * (GL + 1);
     for (int e = threadIdx.x; e < G * (GL + 1); e += DG_THREADS) {
         const int i = e / (GL + 1), l = e % (GL + 1);
@@ -91,95 +106,115 @@ __global__ __launch_bounds__(DG_THREADS) void lo_off_vjp_kernel(LeftVjpArgs v, i
     __shared__ double2 sx[G][PB + 1];
     __shared__ double2 sw[G][PB + 1];
     __shared__ double2 st[G][PB + 1];
-    __shared__ double2 sacc[GL + 1][DG_THREADS];  // lane t's dA row (l < GL) and dB (l == GL)
+    __shared__ double2 sacc[GL + 1][DG_THREADS];
     const LeftArgs &a = v.a;
     const int t = threadIdx.x;
     for (int e = t; e < GL * GL; e += DG_THREADS)
         sA[e / GL][e % GL] = a.A[src_index<L, REORDER>(e / GL) * GL + src_index<L, REORDER>(e % GL)];
     if (t < GL) sB[t] = a.B[src_index<L, REORDER>(t)];
+    const double2 z = make_double2(0.0, 0.0);
+    double2 acc[GL + 1];
 #pragma unroll
-    for (int l = 0; l <= GL; ++l) sacc[l][t] = make_double2(0.0, 0.0);
+    for (int l = 0; l <= GL; ++l) acc[l] = z;
     __syncthreads();
     const int64_t P = a.t.P, C = a.C;
     const int c0 = a.c0;
-    const double2 z = make_double2(0.0, 0.0);
+    constexpr bool AHEAD = MT <= 3;  // every pivot's inputs in one round trip (22 registers each)
 
     for (int it = 0; it < iters; ++it) {
         const LoLane<MT> l = lo_lane<MT, PB>(a, count, start, int64_t(it) * gridDim.x + blockIdx.x);
         const int runmask = lo_runmask<MT>(a, l);
         const bool up_m = l.bm + 1 < c0, up_n = l.bn + 1 < c0;
-        const double2 g0 = l.act ? a.t.inO[l.gs * C + l.pos] : z;
+        const double sbm = a.t.sq[l.bm], sbn = a.t.sq[l.bn], sbm1 = a.t.sq[l.bm + 1], sbn1 = a.t.sq[l.bn + 1];
+        auto fetch = [&](int d, LoIn &q) {
+            lo_clear(q);
+            if (!(runmask >> d & 1) || l.i < 2 * d) return;
+            const int pd = l.p[d];
+            // the input this lane's column carries (as lo_off_kernel reads it)
+            if (l.i == 2 * d) {
+                q.x = a.t.inO[l.gs * C + l.pos];
+                q.sx = a.t.sq[pd + 1];
+            } else if (l.pm > 0) {
+                if (d == 0) {
+                    q.x = a.t.inO[(l.i * P + l.gs) * C + l.pos];
+                } else if (l.i == 2 * d + 1) {
+                    q.x = a.t.arr2[(a.t.off2[d] + l.f - l.sm) * C + l.pos];
+                } else {
+                    const int64_t en = (a.t.off11[d] + (l.m - d - 1) * a.t.len[d] + l.f - l.sm) * C + l.pos;
+                    q.x = (l.i & 1) ? a.t.a1010[en] : a.t.a1001[en];
+                }
+                q.sx = a.t.sq[l.pm];
+            }
+            // the adjoint of this lane's output, where lo_off_kernel wrote it
+            const double2 *src = nullptr;
+            int kk = 0;
+            if (l.i == 2 * d + 1) {
+                src = v.adO + l.fw * C;  // arr0[p + e_d]
+                kk = pd + 1;
+            } else if (l.i == 2 * d) {
+                if (pd + 2 < a.t.cut[d]) {
+                    src = d == 0 ? v.adO + (P + l.fw) * C : v.ad2 + (a.t.off2[d] + l.f) * C;
+                    kk = pd + 2;
+                }
+            } else if (l.pm + 1 < l.cm) {
+                if (d == 0) {
+                    src = v.adO + ((l.i ^ 1) * P + l.fw) * C;
+                } else {
+                    const int64_t e = (a.t.off11[d] + (l.m - d - 1) * a.t.len[d] + l.f) * C;
+                    src = (l.i & 1) ? v.ad1001 + e : v.ad1010 + e;
+                }
+                kk = l.pm + 1;
+            }
+            if (src) {
+                lo_load_adjoints(src, l.pos, c0, up_m, up_n, q);
+                q.K = a.t.sq[kk];
+                q.rK = a.t.rsq[kk];
+            }
+            const double2 *pb = a.piv + (d * P + l.gs) * C;  // arr1[2d, p] block: the pivot
+            q.pv = pb[l.pos];
+            if (l.bm > 0) q.pvm = pb[l.pos - c0];
+            if (l.bn > 0) q.pvn = pb[l.pos - 1];
+        };
+        LoIn in[AHEAD ? MT : 1];
+        if (AHEAD) {
+#pragma unroll
+            for (int d = 0; d < MT; ++d) fetch(d, in[d]);
+        }
         double2 gbar0 = z;  // this lane's share of arr0[p]'s adjoint (lanes 2d)
 #pragma unroll
         for (int d = 0; d < MT; ++d) {
             const bool run = (runmask >> d & 1) && l.i >= 2 * d;
-            const int pd = l.p[d];
-            double2 x = z, wo = z, wm = z, wn = z;
+            if (!AHEAD) fetch(d, in[0]);
+            const LoIn &q = in[AHEAD ? d : 0];
+            double2 wo = z, term = z;
             if (run) {
-                // the input this lane's column carries (as lo_off_kernel reads it)
-                if (l.i == 2 * d) {
-                    x = cscale_promoted(g0, a.t.sq[pd + 1]);
-                } else if (l.pm > 0) {
-                    double2 xr;
-                    if (d == 0) {
-                        xr = a.t.inO[(l.i * P + l.gs) * C + l.pos];
-                    } else if (l.i == 2 * d + 1) {
-                        xr = a.t.arr2[(a.t.off2[d] + l.f - l.sm) * C + l.pos];
-                    } else {
-                        const int64_t en = (a.t.off11[d] + (l.m - d - 1) * a.t.len[d] + l.f - l.sm) * C + l.pos;
-                        xr = (l.i & 1) ? a.t.a1010[en] : a.t.a1001[en];
-                    }
-                    x = cscale_promoted(xr, a.t.sq[l.pm]);
-                }
-                // the adjoint of this lane's output, where lo_off_kernel wrote it
-                const double2 *src = nullptr;
-                int kk = 0;
-                if (l.i == 2 * d + 1) {
-                    src = v.adO + l.fw * C;  // arr0[p + e_d]
-                    kk = pd + 1;
-                } else if (l.i == 2 * d) {
-                    if (pd + 2 < a.t.cut[d]) {
-                        src = d == 0 ? v.adO + (P + l.fw) * C : v.ad2 + (a.t.off2[d] + l.f) * C;
-                        kk = pd + 2;
-                    }
-                } else if (l.pm + 1 < l.cm) {
-                    if (d == 0) {
-                        src = v.adO + ((l.i ^ 1) * P + l.fw) * C;
-                    } else {
-                        const int64_t e = (a.t.off11[d] + (l.m - d - 1) * a.t.len[d] + l.f) * C;
-                        src = (l.i & 1) ? v.ad1001 + e : v.ad1010 + e;
-                    }
-                    kk = l.pm + 1;
-                }
-                if (src) lo_out_adjoints(src, nullptr, l.pos, c0, up_m, up_n, a.t.sq[kk], a.t.rsq[kk], wo, wm, wn);
+                wo = cdiv_by(q.o, q.K, q.rK);
+                term = lo_piv_term<L>(sA, sB, l.i + 2, wo, cdiv_by(q.om, q.K, q.rK), cdiv_by(q.on, q.K, q.rK), up_m, up_n, sbm1, sbn1);
             }
-            double2 term = z;
-            if (run) term = lo_piv_term<L>(sA, sB, l.i + 2, wo, wm, wn, up_m, up_n, a.t.sq[l.bm + 1], a.t.sq[l.bn + 1]);
             if (l.lane_ok) {
-                sx[l.i][l.slot] = x;
+                sx[l.i][l.slot] = run && (l.i == 2 * d || l.pm > 0) ? cscale_promoted(q.x, q.sx) : z;
                 sw[l.i][l.slot] = wo;
                 st[l.i][l.slot] = term;
             }
             __syncthreads();
             if (run) {
-                const int64_t pb = (d * P + l.gs) * C + l.pos;  // arr1[2d, p] block: the pivot
-                sacc[GL][t] = cfma(wo, a.piv[pb], sacc[GL][t]);
-                if (l.bm > 0) sacc[0][t] = cfma(wo, cscale_promoted(a.piv[pb - c0], a.t.sq[l.bm]), sacc[0][t]);
-                if (l.bn > 0) sacc[1][t] = cfma(wo, cscale_promoted(a.piv[pb - 1], a.t.sq[l.bn]), sacc[1][t]);
+                acc[GL] = cfma(wo, q.pv, acc[GL]);
+                if (l.bm > 0) acc[0] = cfma(wo, cscale_promoted(q.pvm, sbm), acc[0]);
+                if (l.bn > 0) acc[1] = cfma(wo, cscale_promoted(q.pvn, sbn), acc[1]);
 #pragma unroll
-                for (int j = 2 * d; j < G; ++j) sacc[j + 2][t] = cfma(wo, sx[j][l.slot], sacc[j + 2][t]);
+                for (int j = 2 * d; j < G; ++j) acc[j + 2] = cfma(wo, sx[j][l.slot], acc[j + 2]);
                 // lane i as column j = i: sum_r w_r A_r,j+2
                 double2 s = z;
 #pragma unroll
                 for (int r = 2 * d; r < G; ++r) s = cfma(sw[r][l.slot], sA[r + 2][l.i + 2], s);
                 if (l.i == 2 * d) {
-                    gbar0 = caxpy(a.t.sq[pd + 1], s, gbar0);
+                    gbar0 = caxpy(q.sx, s, gbar0);
                     double2 gb = z;
 #pragma unroll
                     for (int r = 2 * d; r < G; ++r) gb = cadd(gb, st[r][l.slot]);
-                    v.adP[pb] = gb;
+                    v.adP[(d * P + l.gs) * C + l.pos] = gb;
                 } else if (l.pm > 0) {
-                    const double2 raw = cscale_promoted(s, a.t.sq[l.pm]);
+                    const double2 raw = cscale_promoted(s, q.sx);
                     if (d == 0) {
                         v.adO[(l.i * P + l.gs) * C + l.pos] = raw;
                     } else if (l.i == 2 * d + 1) {
@@ -193,20 +228,20 @@ __global__ __launch_bounds__(DG_THREADS) void lo_off_vjp_kernel(LeftVjpArgs v, i
                     }
                 }
             }
-            __syncthreads();
+            lds_barrier();
         }
         // the off-diagonal pivots' share of arr0[p]'s adjoint, completed by lo_diag_vjp_kernel
         if (l.lane_ok) sx[l.i][l.slot] = gbar0;
-        __syncthreads();
+        lds_barrier();
         if (l.act && l.i == 0) {
             double2 gb = z;
 #pragma unroll
             for (int d = 0; d < MT; ++d) gb = cadd(gb, sx[2 * d][l.slot]);
             v.adO[l.gs * C + l.pos] = gb;
         }
-        __syncthreads();
+        lds_barrier();
     }
-    lo_vjp_flush<MT>(v.part, sacc);
+    lo_vjp_flush<MT>(v.part, acc, sacc);
 }
 
 // Diagonal pivots of one weight in reverse (use_diag_pivot,
@@ -226,12 +261,13 @@ __global__ __launch_bounds__(DG_THREADS) void lo_diag_vjp_kernel(LeftVjpArgs v, 
     for (int e = t; e < GL * GL; e += DG_THREADS)
         sA[e / GL][e % GL] = a.A[src_index<L, REORDER>(e / GL) * GL + src_index<L, REORDER>(e % GL)];
     if (t < GL) sB[t] = a.B[src_index<L, REORDER>(t)];
+    const double2 z = make_double2(0.0, 0.0);
+    double2 acc[GL + 1];
 #pragma unroll
-    for (int l = 0; l <= GL; ++l) sacc[l][t] = make_double2(0.0, 0.0);
+    for (int l = 0; l <= GL; ++l) acc[l] = z;
     __syncthreads();
     const int64_t P = a.t.P, C = a.C;
     const int c0 = a.c0;
-    const double2 z = make_double2(0.0, 0.0);
 
     for (int it = 0; it < iters; ++it) {
         const LoLane<MT> l = lo_lane<MT, PB>(a, count, start, int64_t(it) * gridDim.x + blockIdx.x);
@@ -240,21 +276,41 @@ __global__ __launch_bounds__(DG_THREADS) void lo_diag_vjp_kernel(LeftVjpArgs v, 
         const bool diag = l.act && (a.t.cut[0] == 1 || l.p[0] < a.t.cut[0] - 1);
         const bool dwrite = diag && l.pm + 1 < l.cm && (l.i != 1 || l.p[0] + 2 < a.t.cut[0]);
         const int64_t base = l.gs * C + l.pos;
-        double2 g0 = z, gm = z, gn = z, x = z, wo = z, wm = z, wn = z;
+        const double sbm = a.t.sq[l.bm], sbn = a.t.sq[l.bn], sbm1 = a.t.sq[l.bm + 1], sbn1 = a.t.sq[l.bn + 1], spm = a.t.sq[l.pm];
+        // q.pv, pvm, pvn: the pivot is the arr0 block of p; e: the off-diagonal
+        // pivot m of p's share for arr1[2m, p], beside consumer p + e_m's diagonal pivot
+        LoIn q, e;
+        lo_clear(q);
+        lo_clear(e);
+        double2 own = z, ct = z;
         if (l.act) {
-            g0 = a.t.inO[base];
-            if (l.bm > 0) gm = a.t.inO[base - c0];
-            if (l.bn > 0) gn = a.t.inO[base - 1];
+            q.pv = a.t.inO[base];
+            if (l.bm > 0) q.pvm = a.t.inO[base - c0];
+            if (l.bn > 0) q.pvn = a.t.inO[base - 1];
+            if (l.i == 0) {
+                own = v.adO[base];
+                ct = v.cot[int64_t(l.pos) * P + l.f];
+            }
         }
-        if (diag && l.pm > 0) x = cscale_promoted(a.t.inD[(l.i * P + l.gs) * C + l.pos], a.t.sq[l.pm]);
+        if (diag && l.pm > 0) q.x = a.t.inD[(l.i * P + l.gs) * C + l.pos];
+        const bool ext = dwrite && !(l.i & 1) && (runmask >> l.m & 1);
         if (dwrite) {
-            // consumer p + e_m's diagonal pivot, plus the off-diagonal pivot m of p for arr1[2m, p]
-            const double2 *ext = (!(l.i & 1) && (runmask >> l.m & 1)) ? v.adP + (l.m * P + l.gs) * C : nullptr;
-            lo_out_adjoints(v.adD + ((l.i ^ 1) * P + l.fw) * C, ext, l.pos, c0, up_m, up_n, a.t.sq[l.pm + 1], a.t.rsq[l.pm + 1], wo,
-                            wm, wn);
+            lo_load_adjoints(v.adD + ((l.i ^ 1) * P + l.fw) * C, l.pos, c0, up_m, up_n, q);
+            q.K = a.t.sq[l.pm + 1];
+            q.rK = a.t.rsq[l.pm + 1];
         }
-        double2 term = z;
-        if (dwrite) term = lo_piv_term<L>(sA, sB, l.i + 2, wo, wm, wn, up_m, up_n, a.t.sq[l.bm + 1], a.t.sq[l.bn + 1]);
+        if (ext) lo_load_adjoints(v.adP + (l.m * P + l.gs) * C, l.pos, c0, up_m, up_n, e);
+        if (ext) {
+            q.o = cadd(q.o, e.o);
+            q.om = cadd(q.om, e.om);
+            q.on = cadd(q.on, e.on);
+        }
+        const double2 x = diag && l.pm > 0 ? cscale_promoted(q.x, spm) : z;
+        double2 wo = z, term = z;
+        if (dwrite) {
+            wo = cdiv_by(q.o, q.K, q.rK);
+            term = lo_piv_term<L>(sA, sB, l.i + 2, wo, cdiv_by(q.om, q.K, q.rK), cdiv_by(q.on, q.K, q.rK), up_m, up_n, sbm1, sbn1);
+        }
         if (l.lane_ok) {
             sx[l.i][l.slot] = x;
             sw[l.i][l.slot] = wo;
@@ -262,28 +318,28 @@ __global__ __launch_bounds__(DG_THREADS) void lo_diag_vjp_kernel(LeftVjpArgs v, 
         }
         __syncthreads();
         if (diag) {
-            sacc[GL][t] = cfma(wo, g0, sacc[GL][t]);
-            if (l.bm > 0) sacc[0][t] = cfma(wo, cscale_promoted(gm, a.t.sq[l.bm]), sacc[0][t]);
-            if (l.bn > 0) sacc[1][t] = cfma(wo, cscale_promoted(gn, a.t.sq[l.bn]), sacc[1][t]);
+            acc[GL] = cfma(wo, q.pv, acc[GL]);
+            if (l.bm > 0) acc[0] = cfma(wo, cscale_promoted(q.pvm, sbm), acc[0]);
+            if (l.bn > 0) acc[1] = cfma(wo, cscale_promoted(q.pvn, sbn), acc[1]);
 #pragma unroll
-            for (int j = 0; j < G; ++j) sacc[j + 2][t] = cfma(wo, sx[j][l.slot], sacc[j + 2][t]);
+            for (int j = 0; j < G; ++j) acc[j + 2] = cfma(wo, sx[j][l.slot], acc[j + 2]);
             double2 s = z;
 #pragma unroll
             for (int r = 0; r < G; ++r) s = cfma(sw[r][l.slot], sA[r + 2][l.i + 2], s);
-            if (l.pm > 0) v.adD[(l.i * P + l.gs) * C + l.pos] = cscale_promoted(s, a.t.sq[l.pm]);
+            if (l.pm > 0) v.adD[(l.i * P + l.gs) * C + l.pos] = cscale_promoted(s, spm);
         }
         if (l.act && l.i == 0) {
             // cotangent + off-diagonal share + the diagonal pivot's block terms
-            double2 gb = cadd(v.cot[int64_t(l.pos) * P + l.f], v.adO[base]);
+            double2 gb = cadd(make_double2(ct.x, v.gsign * ct.y), own);
             if (diag) {
 #pragma unroll
                 for (int r = 0; r < G; ++r) gb = cadd(gb, st[r][l.slot]);
             }
             v.adO[base] = gb;
         }
-        __syncthreads();
+        lds_barrier();
     }
-    lo_vjp_flush<MT>(v.part, sacc);
+    lo_vjp_flush<MT>(v.part, acc, sacc);
 }
 
 // The zero-detection block in reverse (singleLeftoverMode_amps.py:330-341):
@@ -341,7 +397,7 @@ __global__ __launch_bounds__(1024) void lo_init_vjp_kernel(LeftVjpArgs v, int nb
                 sw[k - 2] = cfma(cscale_promoted(w, a.t.sq[k - 1]), A00, sw[k - 2]);
             }
         }
-        *v.dc = sw[0];
+        *v.dc = make_double2(sw[0].x, v.gsign * sw[0].y);
     }
     // block sums of the column terms, in a fixed tree
     double2 *prow = v.part + int64_t(nblk) * GL * (GL + 1);

@@ -22,7 +22,8 @@ import torch
 from .. import _lib
 from .strategies import C128, _ptr, _shape_arr, _stream, _workspace, as_device_c128
 
-__all__ = ["diagonal_hip", "diagonal_vjp_hip", "input_validation", "leftover_hip", "leftover_vjp_hip"]
+__all__ = ["diagonal_hip", "diagonal_vjp_hip", "input_validation", "leftover_grad_hip", "leftover_hip",
+           "leftover_vjp_hip"]
 
 
 def input_validation(A, rtol: float = 1e-05, atol: float = 1e-08) -> bool:
@@ -106,6 +107,11 @@ def diagonal_vjp_hip(A, B, G0, cutoffs, dLdG, reordered: bool = False):
     return G, dA, dB, dc
 
 
+# The largest forward workspace that a tracked call keeps for its backward; a
+# larger one is computed again there.
+LEFTOVER_KEEP_BYTES = 64 << 20
+
+
 def leftover_hip(A, b, c, output_cutoff: int, pnr_cutoffs, reordered: bool = True, rtol: float = 1e-05,
                  atol: float = 1e-08) -> torch.Tensor:
     """out[m, n, k] = G[(m, k), (n, k)]: mode 0's density matrix (m, n <=
@@ -113,6 +119,11 @@ def leftover_hip(A, b, c, output_cutoff: int, pnr_cutoffs, reordered: bool = Tru
     photons.  (A, b, c) in the [modes..., modes...] order when ``reordered``
     (reorder_AB_bargmann, backend_numpy.py:367-375), else [mode0, mode0, mode1,
     mode1, ...].  Raises ValueError as inputValidation.py:103-118 does."""
+    return _leftover(A, b, c, output_cutoff, pnr_cutoffs, reordered, rtol, atol)[0]
+
+
+def _leftover(A, b, c, output_cutoff, pnr_cutoffs, reordered, rtol=1e-05, atol=1e-08):
+    """``leftover_hip`` and the workspace that it filled."""
     A, b, c = as_device_c128(A), as_device_c128(b), as_device_c128(c)
     input_validation(A, rtol=rtol, atol=atol)
     if A.shape[0] != b.shape[0]:
@@ -137,7 +148,28 @@ def leftover_hip(A, b, c, output_cutoff: int, pnr_cutoffs, reordered: bool = Tru
         _ptr(out), _ptr(ws), 0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_1leftover")
-    return out
+    return out, ws
+
+
+def leftover_grad_hip(A, b, c, output_cutoff: int, pnr_cutoffs, ws, grad, reordered: bool = True):
+    """(dL/dA, dL/db, dL/dc) in torch's convention for ``grad`` = dL/d(conj out),
+    from the workspace ``ws`` that the forward of the same triple filled: the
+    reverse sweep of ``leftover_vjp_hip`` without a second forward."""
+    A, b, c, g = as_device_c128(A), as_device_c128(b), as_device_c128(c), as_device_c128(grad)
+    pnr = tuple(int(k) for k in pnr_cutoffs)
+    o = int(output_cutoff)
+    if tuple(g.shape) != (o + 1, o + 1, *(k + 1 for k in pnr)):
+        raise ValueError("the gradient must have the shape of the output")
+    dA, db, dc = torch.empty_like(A), torch.empty_like(b), torch.empty((), dtype=C128, device=A.device)
+    s = _shape_arr(pnr)
+    L = _lib.load()
+    gws = _workspace(L.mm_hermite_1leftover_grad_workspace(o, s.ctypes.data, len(pnr)))
+    rc = L.mm_hermite_1leftover_grad(
+        _ptr(A), _ptr(b), _ptr(c), o, s.ctypes.data, len(pnr), int(bool(reordered)), _ptr(ws), ws.numel(), _ptr(g),
+        _ptr(dA), _ptr(db), _ptr(dc), _ptr(gws), 0 if gws is None else gws.numel(), _stream(),
+    )
+    _lib.check(rc, "mm_hermite_1leftover_grad")
+    return dA, db, dc
 
 
 def leftover_vjp_hip(A, b, c, output_cutoff: int, pnr_cutoffs, dLdout, reordered: bool = True):

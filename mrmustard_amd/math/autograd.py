@@ -112,15 +112,21 @@ class HermiteDiagonal(torch.autograd.Function):
 class HermiteLeftover(torch.autograd.Function):
     """out = hermite_renormalized_1leftoverMode(A, b, c, output_cutoff,
     pnr_cutoffs) with the reverse-sweep VJP (the reference's jax custom VJP
-    pair, jax_vjps/hermite.py:343-445).  The backward recomputes the forward
-    together with the VJP (``leftover_vjp_hip``), so only (A, b, c) are kept."""
+    pair, jax_vjps/hermite.py:343-445).  The forward's intermediate blocks are
+    kept for the backward up to ``LEFTOVER_KEEP_BYTES`` (a (20, 20, 15, 15)
+    output: 16 MB; its second forward took a quarter of a training step);
+    beyond that only (A, b, c) are kept and the backward recomputes them
+    (``leftover_vjp_hip``)."""
 
     @staticmethod
     def forward(ctx, A, b, c, output_cutoff, pnr_cutoffs, reordered):
         from ..lattice import compact_fock as cf
 
-        out = cf.leftover_hip(A, b, c, output_cutoff, pnr_cutoffs, reordered=reordered)
-        ctx.save_for_backward(A, b, c)
+        out, ws = cf._leftover(A, b, c, output_cutoff, pnr_cutoffs, reordered)
+        if ws.numel() <= cf.LEFTOVER_KEEP_BYTES:
+            ctx.save_for_backward(A, b, c, ws)
+        else:
+            ctx.save_for_backward(A, b, c)
         ctx.args = (int(output_cutoff), tuple(int(k) for k in pnr_cutoffs), bool(reordered))
         return out
 
@@ -128,7 +134,10 @@ class HermiteLeftover(torch.autograd.Function):
     def backward(ctx, grad):
         from ..lattice import compact_fock as cf
 
-        A, b, c = ctx.saved_tensors
+        A, b, c, *kept = ctx.saved_tensors
         o, pnr, reordered = ctx.args
-        _, dA, db, dc = cf.leftover_vjp_hip(*st.conj_triple(A, b, c), o, pnr, grad, reordered=reordered)
+        if kept:
+            dA, db, dc = cf.leftover_grad_hip(A, b, c, o, pnr, kept[0], grad, reordered=reordered)
+        else:
+            _, dA, db, dc = cf.leftover_vjp_hip(*st.conj_triple(A, b, c), o, pnr, grad, reordered=reordered)
         return dA.reshape(A.shape), db.reshape(b.shape), dc.reshape(c.shape), None, None, None
