@@ -20,7 +20,7 @@ import numpy as np
 import torch
 
 from .. import _lib
-from .strategies import C128, _ptr, _shape_arr, _stream, _workspace, as_device_c128
+from .strategies import C128, _addr, _ptr, _shape_arr, _stream, _workspace, as_device_c128
 
 __all__ = ["diagonal_hip", "diagonal_vjp_hip", "input_validation", "leftover_grad_hip", "leftover_hip",
            "leftover_vjp_hip"]
@@ -68,9 +68,9 @@ def diagonal_hip(A, B, G0, cutoffs, reordered: bool = False, rtol: float = 1e-05
         return G
     s = _shape_arr(cutoffs)
     L = _lib.load()
-    ws = _workspace(L.mm_hermite_diagonal_workspace(s.ctypes.data, M, nb))
+    ws = _workspace(L.mm_hermite_diagonal_workspace(_addr(s), M, nb))
     rc = L.mm_hermite_diagonal(
-        _ptr(A), _ptr(B), _ptr(G0), int(G0.numel() > 1), s.ctypes.data, M, nb, int(bool(reordered)),
+        _ptr(A), _ptr(B), _ptr(G0), int(G0.numel() > 1), _addr(s), M, nb, int(bool(reordered)),
         _ptr(G), _ptr(ws), 0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_diagonal")
@@ -98,9 +98,9 @@ def diagonal_vjp_hip(A, B, G0, cutoffs, dLdG, reordered: bool = False):
     dc = torch.empty((), dtype=C128, device=A.device)
     s = _shape_arr(cutoffs)
     L = _lib.load()
-    ws = _workspace(L.mm_hermite_diagonal_vjp_workspace(s.ctypes.data, M))
+    ws = _workspace(L.mm_hermite_diagonal_vjp_workspace(_addr(s), M))
     rc = L.mm_hermite_diagonal_vjp(
-        _ptr(A), _ptr(B), _ptr(G0), s.ctypes.data, M, int(bool(reordered)), _ptr(g), _ptr(G), _ptr(dA), _ptr(dB), _ptr(dc),
+        _ptr(A), _ptr(B), _ptr(G0), _addr(s), M, int(bool(reordered)), _ptr(g), _ptr(G), _ptr(dA), _ptr(dB), _ptr(dc),
         _ptr(ws), 0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_diagonal_vjp")
@@ -142,9 +142,9 @@ def _leftover(A, b, c, output_cutoff, pnr_cutoffs, reordered, rtol=1e-05, atol=1
     out = torch.empty((o + 1, o + 1, *(k + 1 for k in pnr)), dtype=C128, device=A.device)
     s = _shape_arr(pnr)
     L = _lib.load()
-    ws = _workspace(L.mm_hermite_1leftover_workspace(o, s.ctypes.data, M - 1))
+    ws = _workspace(L.mm_hermite_1leftover_workspace(o, _addr(s), M - 1))
     rc = L.mm_hermite_1leftover(
-        _ptr(A), _ptr(b), _ptr(c), o, s.ctypes.data, M - 1, int(bool(reordered)),
+        _ptr(A), _ptr(b), _ptr(c), o, _addr(s), M - 1, int(bool(reordered)),
         _ptr(out), _ptr(ws), 0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_1leftover")
@@ -163,9 +163,9 @@ def leftover_grad_hip(A, b, c, output_cutoff: int, pnr_cutoffs, ws, grad, reorde
     dA, db, dc = torch.empty_like(A), torch.empty_like(b), torch.empty((), dtype=C128, device=A.device)
     s = _shape_arr(pnr)
     L = _lib.load()
-    gws = _workspace(L.mm_hermite_1leftover_grad_workspace(o, s.ctypes.data, len(pnr)))
+    gws = _workspace(L.mm_hermite_1leftover_grad_workspace(o, _addr(s), len(pnr)))
     rc = L.mm_hermite_1leftover_grad(
-        _ptr(A), _ptr(b), _ptr(c), o, s.ctypes.data, len(pnr), int(bool(reordered)), _ptr(ws), ws.numel(), _ptr(g),
+        _ptr(A), _ptr(b), _ptr(c), o, _addr(s), len(pnr), int(bool(reordered)), _ptr(ws), ws.numel(), _ptr(g),
         _ptr(dA), _ptr(db), _ptr(dc), _ptr(gws), 0 if gws is None else gws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_1leftover_grad")
@@ -198,9 +198,9 @@ def leftover_vjp_hip(A, b, c, output_cutoff: int, pnr_cutoffs, dLdout, reordered
     dc = torch.empty((), dtype=C128, device=A.device)
     s = _shape_arr(pnr)
     L = _lib.load()
-    ws = _workspace(L.mm_hermite_1leftover_vjp_workspace(o, s.ctypes.data, M - 1))
+    ws = _workspace(L.mm_hermite_1leftover_vjp_workspace(o, _addr(s), M - 1))
     rc = L.mm_hermite_1leftover_vjp(
-        _ptr(A), _ptr(b), _ptr(c), o, s.ctypes.data, M - 1, int(bool(reordered)), _ptr(g), _ptr(out), _ptr(dA), _ptr(db),
+        _ptr(A), _ptr(b), _ptr(c), o, _addr(s), M - 1, int(bool(reordered)), _ptr(g), _ptr(out), _ptr(dA), _ptr(db),
         _ptr(dc), _ptr(ws), 0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_1leftover_vjp")

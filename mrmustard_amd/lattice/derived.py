@@ -29,7 +29,7 @@ import torch
 from .. import _lib
 from ..contraction import zgemm_batched_hip
 from ..settings import settings
-from .strategies import C128, _ptr, _shape_arr, _stream, _workspace, as_device_c128
+from .strategies import C128, _addr, _ptr, _shape_arr, _stream, _workspace, as_device_c128
 
 FUSE_MIN_AMPS = 1 << 20  # lattice entries per triple from which fock_array_derived fuses by default
 
@@ -77,9 +77,9 @@ def _fused_batch(A3, b3, c3, full_shape, n):
     K = pymath.prod(full_shape[n:])
     w = c3.reshape(nb, K).contiguous()
     out = torch.empty((nb,) + tuple(full_shape[:n]), dtype=C128, device=A3.device)
-    ws = _workspace(L.mm_hermite_batch_fwd_contract_workspace(s.ctypes.data, D))
+    ws = _workspace(L.mm_hermite_batch_fwd_contract_workspace(_addr(s), D))
     rc = L.mm_hermite_batch_fwd_contract(
-        _ptr(A3.contiguous()), _ptr(b3.contiguous()), _ptr(ones), nb, s.ctypes.data, D, n, _ptr(w), 1, K, _ptr(out),
+        _ptr(A3.contiguous()), _ptr(b3.contiguous()), _ptr(ones), nb, _addr(s), D, n, _ptr(w), 1, K, _ptr(out),
         _ptr(ws), 0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_batch_fwd_contract")

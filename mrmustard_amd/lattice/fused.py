@@ -32,7 +32,7 @@ import torch
 from .. import _lib
 from ..contraction import contract
 from ..settings import settings
-from .strategies import C128, _ptr, _shape_arr, _stream, _workspace, as_device_c128
+from .strategies import C128, _addr, _ptr, _shape_arr, _stream, _workspace, as_device_c128
 
 __all__ = ["fock_contract"]
 
@@ -114,9 +114,9 @@ def fock_contract(A, b, c, shape, idx1, array, idx2, idx_out, fused: bool | None
     if nb > 0:
         L = _lib.load()
         s = _shape_arr(shp)
-        ws = _workspace(L.mm_hermite_batch_fwd_contract_workspace(s.ctypes.data, D))
+        ws = _workspace(L.mm_hermite_batch_fwd_contract_workspace(_addr(s), D))
         rc = L.mm_hermite_batch_fwd_contract(
-            _ptr(Ap), _ptr(bp), _ptr(cp), nb, s.ctypes.data, D, len(kept), _ptr(Wm), M, 0, _ptr(out),
+            _ptr(Ap), _ptr(bp), _ptr(cp), nb, _addr(s), D, len(kept), _ptr(Wm), M, 0, _ptr(out),
             _ptr(ws), 0 if ws is None else ws.numel(), _stream(),
         )
         _lib.check(rc, "mm_hermite_batch_fwd_contract")

@@ -26,8 +26,8 @@ conjugated, and dA is returned symmetrised, (M + M^T)/2.
 from __future__ import annotations
 
 import cmath
-import ctypes
 import math as pymath
+from array import array
 
 import numpy as np
 import torch
@@ -52,13 +52,16 @@ C128 = torch.complex128
 
 
 def _device() -> torch.device:
-    if not torch.cuda.is_available():
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
         raise RuntimeError("mrmustard_amd needs a ROCm GPU: torch.cuda.is_available() is False")
     return torch.device("cuda", torch.cuda.current_device())
 
 
 def as_device_c128(x) -> torch.Tensor:
     """complex128, contiguous, on the current GPU (copies only when needed)."""
+    if (isinstance(x, torch.Tensor) and x.dtype == C128 and x.is_cuda and x.is_contiguous() and not x.is_conj() and not x.is_neg()
+            and x.device.index == torch.cuda.current_device()):
+        return x
     dev = _device()
     if isinstance(x, torch.Tensor):
         t = x
@@ -74,16 +77,21 @@ def as_device_c128(x) -> torch.Tensor:
     return torch.as_tensor(np.asarray(x, dtype=np.complex128), device=dev).contiguous()
 
 
-def _shape_arr(shape) -> np.ndarray:
-    return np.ascontiguousarray(np.asarray([int(s) for s in shape], dtype=np.int64))
+def _shape_arr(shape) -> array:
+    return array("q", [int(s) for s in shape])
+
+
+def _addr(s: array) -> int:
+    """Address of a shape; the caller holds the array during the call."""
+    return s.buffer_info()[0]
 
 
 def _ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream() -> int:
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _workspace(nbytes: int) -> torch.Tensor | None:
@@ -121,9 +129,9 @@ def _fwd(shape, A, b, c, stable: bool, out=None) -> torch.Tensor:
     shape = _check_shape(shape, D)
     G = _out_tensor(out, shape)
     s = _shape_arr(shape)
-    ws = _workspace(L.mm_hermite_fwd_workspace(s.ctypes.data, D, int(stable)))
+    ws = _workspace(L.mm_hermite_fwd_workspace(_addr(s), D, int(stable)))
     rc = L.mm_hermite_fwd(
-        _ptr(A), _ptr(b), _ptr(c), s.ctypes.data, D, int(stable), _ptr(G), _ptr(ws), 0 if ws is None else ws.numel(), _stream()
+        _ptr(A), _ptr(b), _ptr(c), _addr(s), D, int(stable), _ptr(G), _ptr(ws), 0 if ws is None else ws.numel(), _stream()
     )
     _lib.check(rc, "mm_hermite_fwd")
     return G
@@ -151,9 +159,9 @@ def vanilla_batch_hip(shape, A, b, c, stable: bool = False, out=None) -> torch.T
     if B == 0:
         return G
     s = _shape_arr(shape)
-    ws = _workspace(L.mm_hermite_batch_fwd_workspace(B, s.ctypes.data, D, int(stable)))
+    ws = _workspace(L.mm_hermite_batch_fwd_workspace(B, _addr(s), D, int(stable)))
     rc = L.mm_hermite_batch_fwd(
-        _ptr(A), _ptr(b), _ptr(c), B, s.ctypes.data, D, int(stable), _ptr(G), _ptr(ws), 0 if ws is None else ws.numel(), _stream()
+        _ptr(A), _ptr(b), _ptr(c), B, _addr(s), D, int(stable), _ptr(G), _ptr(ws), 0 if ws is None else ws.numel(), _stream()
     )
     _lib.check(rc, "mm_hermite_batch_fwd")
     return G
@@ -170,9 +178,9 @@ def vanilla_vjp_hip(G, c, dLdG):
     dA = torch.empty((D, D), dtype=C128, device=G.device)
     db = torch.empty((D,), dtype=C128, device=G.device)
     dc = torch.empty((), dtype=C128, device=G.device)
-    ws = _workspace(L.mm_hermite_vjp_workspace(s.ctypes.data, D))
+    ws = _workspace(L.mm_hermite_vjp_workspace(_addr(s), D))
     rc = L.mm_hermite_vjp(
-        _ptr(G), _ptr(c), _ptr(g), s.ctypes.data, D, _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws), 0 if ws is None else ws.numel(), _stream()
+        _ptr(G), _ptr(c), _ptr(g), _addr(s), D, _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws), 0 if ws is None else ws.numel(), _stream()
     )
     _lib.check(rc, "mm_hermite_vjp")
     return dA, db, dc
@@ -191,9 +199,9 @@ def vanilla_batch_vjp_hip(G, c, dLdG):
     dc = torch.empty((B,), dtype=C128, device=G.device)
     if B == 0:
         return dA, db, dc
-    ws = _workspace(L.mm_hermite_batch_vjp_workspace(B, s.ctypes.data, D))
+    ws = _workspace(L.mm_hermite_batch_vjp_workspace(B, _addr(s), D))
     rc = L.mm_hermite_batch_vjp(
-        _ptr(G), _ptr(c), _ptr(g), B, s.ctypes.data, D, _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws), 0 if ws is None else ws.numel(),
+        _ptr(G), _ptr(c), _ptr(g), B, _addr(s), D, _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws), 0 if ws is None else ws.numel(),
         _stream(),
     )
     _lib.check(rc, "mm_hermite_batch_vjp")
@@ -218,9 +226,9 @@ def vanilla_vjp_grad_hip(G, c, grad, batched: bool = False):
     dc = torch.empty(lead, dtype=C128, device=G.device)
     if B == 0:
         return dA, db, dc
-    ws = _workspace(L.mm_hermite_batch_vjp_workspace(B, s.ctypes.data, D))
+    ws = _workspace(L.mm_hermite_batch_vjp_workspace(B, _addr(s), D))
     rc = L.mm_hermite_batch_vjp_conj(
-        _ptr(G), _ptr(c), _ptr(g), B, s.ctypes.data, D, _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws), 0 if ws is None else ws.numel(),
+        _ptr(G), _ptr(c), _ptr(g), B, _addr(s), D, _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws), 0 if ws is None else ws.numel(),
         _stream(),
     )
     _lib.check(rc, "mm_hermite_batch_vjp_conj")
@@ -252,9 +260,9 @@ def vanilla_fused_hip(shape, A, b, c, dLdG, out=None):
     dA = torch.empty((D, D), dtype=C128, device=G.device)
     db = torch.empty((D,), dtype=C128, device=G.device)
     dc = torch.empty((), dtype=C128, device=G.device)
-    ws = _workspace(L.mm_hermite_fused_workspace(s.ctypes.data, D))
+    ws = _workspace(L.mm_hermite_fused_workspace(_addr(s), D))
     rc = L.mm_hermite_fused(
-        _ptr(A), _ptr(b), _ptr(c), _ptr(g), s.ctypes.data, D, _ptr(G), _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws),
+        _ptr(A), _ptr(b), _ptr(c), _ptr(g), _addr(s), D, _ptr(G), _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws),
         0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_fused")
@@ -276,9 +284,9 @@ def vanilla_batch_fused_hip(shape, A, b, c, dLdG, out=None):
     dc = torch.empty((B,), dtype=C128, device=G.device)
     if B == 0:
         return G, dA, db, dc
-    ws = _workspace(L.mm_hermite_batch_fused_workspace(B, s.ctypes.data, D))
+    ws = _workspace(L.mm_hermite_batch_fused_workspace(B, _addr(s), D))
     rc = L.mm_hermite_batch_fused(
-        _ptr(A), _ptr(b), _ptr(c), _ptr(g), B, s.ctypes.data, D, _ptr(G), _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws),
+        _ptr(A), _ptr(b), _ptr(c), _ptr(g), B, _addr(s), D, _ptr(G), _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws),
         0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_batch_fused")
@@ -306,9 +314,9 @@ def vanilla_vjp_recompute_hip(shape, A, b, c, dLdG):
     dA = torch.empty((D, D), dtype=C128, device=g.device)
     db = torch.empty((D,), dtype=C128, device=g.device)
     dc = torch.empty((), dtype=C128, device=g.device)
-    ws = _workspace(L.mm_hermite_vjp_recompute_workspace(s.ctypes.data, D))
+    ws = _workspace(L.mm_hermite_vjp_recompute_workspace(_addr(s), D))
     rc = L.mm_hermite_vjp_recompute(
-        _ptr(A), _ptr(b), _ptr(c), _ptr(g), s.ctypes.data, D, _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws),
+        _ptr(A), _ptr(b), _ptr(c), _ptr(g), _addr(s), D, _ptr(dA), _ptr(db), _ptr(dc), _ptr(ws),
         0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_vjp_recompute")
@@ -332,9 +340,9 @@ def binomial_hip(local_cutoffs, A, b, c, max_l2, global_cutoff):
     norm = torch.empty((), dtype=torch.float64, device=A.device)
     s = _shape_arr(shape)
     L = _lib.load()
-    ws = _workspace(L.mm_hermite_binomial_workspace(s.ctypes.data, D))
+    ws = _workspace(L.mm_hermite_binomial_workspace(_addr(s), D))
     rc = L.mm_hermite_binomial(
-        _ptr(A), _ptr(b), _ptr(c), s.ctypes.data, D, float("inf") if max_l2 is None else float(max_l2), int(global_cutoff),
+        _ptr(A), _ptr(b), _ptr(c), _addr(s), D, float("inf") if max_l2 is None else float(max_l2), int(global_cutoff),
         _ptr(G), _ptr(norm), _ptr(ws), 0 if ws is None else ws.numel(), _stream(),
     )
     _lib.check(rc, "mm_hermite_binomial")

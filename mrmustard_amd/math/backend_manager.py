@@ -18,6 +18,7 @@ into tensors before the dispatch so that ``.ndim`` exists on all of them.
 from __future__ import annotations
 
 from collections.abc import Sequence
+from math import prod
 from typing import Any
 
 import numpy as np
@@ -125,7 +126,7 @@ class BackendManager:
                 raise ValueError(f"b.shape={tuple(b.shape)} must match batch_shape={batch_shape}")
             if tuple(c.shape[: len(batch_shape)]) != batch_shape:
                 raise ValueError(f"c.shape={tuple(c.shape)} must match batch_shape={batch_shape}")
-            D = int(np.prod(batch_shape))
+            D = prod(batch_shape)
             A = self.reshape(A, (D, *A.shape[-2:]))
             b = self.reshape(b, (D, *b.shape[-1:]))
             c = self.reshape(c, (D,))
@@ -138,7 +139,7 @@ class BackendManager:
         if A.ndim == 2 and b.ndim > 1:  # b-batched case
             batch_shape = tuple(b.shape[:-1])
             check_out_shape(batch_shape)
-            D = int(np.prod(batch_shape))
+            D = prod(batch_shape)
             b = self.reshape(b, (D, *b.shape[-1:]))
             A_broadcast = self.broadcast_to(A, (D, *A.shape))
             c_broadcast = self.broadcast_to(c, (D,))
