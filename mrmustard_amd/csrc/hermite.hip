@@ -231,13 +231,21 @@ int pick_threads(int64_t S, int maxt, int rmax) {
     return best;
 }
 
+// Slabs of up to this many points: one point per thread and no idle waves,
+// which would step through every barrier and keep other triples off the CU.
+// Measured against 512 threads (256 fused at D >= 4) for all of them, kernel time:
+// 2,000 of (8, 8) 56 -> 10 us, 1,000 of (20, 20) 55 -> 17, 500 of (15,)^3 36 -> 21,
+// 500 of (5,)^4 27 -> 15, one (50, 50) 27.5 -> 24.9; fused 2,000 of (8, 8) 89 -> 14,
+// 300 of (50, 50) 82 -> 37, 20 of (100, 100) 76 -> 65 us.
+constexpr int SMALL_SLAB = 384;
+
 // Smallest top level whose sweep fits in LDS with `threads` threads (D >= 2).
 int choose_top(const Shape &S, bool fused, int max_lds, int maxt, int *threads) {
     for (int top = 0; top < S.D; ++top) {
         int T = team_threads(S.st[top], maxt);
         if (top == 0) {
             const int Tr = pick_threads(S.st[0], maxt, rmax_for(kernel_dmax(S.D), fused));
-            if (Tr) T = Tr;
+            if (Tr && S.st[0] > SMALL_SLAB) T = Tr;
         }
         if (S.st[top] > int64_t(8) * 1024 * 1024) continue;
         if (!packed_bits_ok(S, top)) continue;
@@ -250,8 +258,8 @@ int choose_top(const Shape &S, bool fused, int max_lds, int maxt, int *threads) 
     return S.D - 1;
 }
 
-// Forward-only uniform batches of D <= 3 triples whose level-0 slab has
-// LEAN_MIN_S .. LEAN_MAX_S points: one point per thread of a workgroup of up
+// Forward-only uniform batches of D <= 3 triples whose level-0 slab has up to
+// SMALL_SLAB or LEAN_MIN_S .. LEAN_MAX_S points: one point per thread of a workgroup of up
 // to 1024 threads, in lds_block_kernel (about 70 registers: four waves per
 // SIMD).  The fused sweep keeps lds_kernel: its one-point-per-thread variant
 // needs 128 registers with spills and measured slower than two points per
@@ -261,8 +269,9 @@ constexpr int LEAN_MIN_S = 512;
 
 // Launch lds_block_kernel for S if it applies; returns 1 if it does not.
 int launch_lean(const LdsArgs &a0, const Shape &S, bool fused, int64_t B, const DevState *ds, hipStream_t s) {
-    if (fused || S.D < 2 || S.D > 3 || S.st[0] < LEAN_MIN_S || S.st[0] > LEAN_MAX_S || !packed_bits_ok(S, 0)) return 1;
-    const int T = pick_threads(S.st[0], 1024, 1);
+    if (fused || S.D < 2 || S.D > 3 || S.st[0] > LEAN_MAX_S || !packed_bits_ok(S, 0)) return 1;
+    if (S.st[0] > SMALL_SLAB && S.st[0] < LEAN_MIN_S) return 1;  // (200, 400): 145 us in lds_kernel, 147 here
+    const int T = S.st[0] <= SMALL_SLAB ? team_threads(S.st[0], SMALL_SLAB) : pick_threads(S.st[0], 1024, 1);
     if (!T) return 1;
     const int64_t shmem = lds_bytes_rm(S, 0, fused, T / MM_WAVE, 1);
     if (shmem > ds->max_lds) return 1;

@@ -347,7 +347,7 @@ __device__ __forceinline__ void level0_reg(const Job &J, const Team<WAVE> &tm, d
 // `rank`/`tsize` number the participating threads; smode is the ordering
 // between steps: 0 = a single lane (no ordering needed), 1 = one wave,
 // 2 = the team barrier.
-template <int D, bool FUSED, bool WAVE, int L, int NR>
+template <int D, bool FUSED, bool WAVE, int L, int NR, bool AHEAD>
 __device__ __forceinline__ void level_straight(const Job &J, const Team<WAVE> &tm, int rank, int tsize, int smode, double2 *ring,
                                                const uint32_t *kv, const double *sq, const double *rsq, const double2 *bv,
                                                const double2 *A, double2 *G, const double2 *g, Acc<D> &acc) {
@@ -388,11 +388,32 @@ __device__ __forceinline__ void level_straight(const Job &J, const Team<WAVE> &t
         gnext[r] = zero;
         if (VJP && sd > 1) gcur[r] = g[int64_t(S) + q[r]];  // masked where used
     }
+    // AHEAD: a level that one wave sweeps has nothing but its own latency to hide
+    // and reads a step's roots a step ahead (levels of several waves measured 2 to
+    // 4 % slower that way)
+    double sm_a = 0.0, rm_a = 0.0, sm1_a = 0.0;
+    if (AHEAD && smode == 1 && sd > 1) {
+        sm_a = sq[1];
+        rm_a = rsq[1];
+        sm1_a = sq[0];
+    }
     for (int m = 1; m < sd; ++m) {
         double2 *cur = TOP ? ring + (m & 1) * S : ring + m * Sd;
         const double2 *p1 = TOP ? ring + ((m - 1) & 1) * S : ring + (m - 1) * Sd;
-        const double sm = sq[m], rm = rsq[m];
-        const double sm1 = sq[m - 1];
+        double sm, rm, sm1;
+        if (AHEAD && smode == 1) {
+            sm = sm_a;
+            rm = rm_a;
+            sm1 = sm1_a;
+            const int mn = m + 1 < sd ? m + 1 : m;
+            sm_a = sq[mn];
+            rm_a = rsq[mn];
+            sm1_a = sm;
+        } else {
+            sm = sq[m];
+            rm = rsq[m];
+            sm1 = sq[m - 1];
+        }
         const double2 cLL = cscale_promoted(aLL, sm1);
         const int64_t gbase = int64_t(m) * Sd;
         if (VJP && m + 1 < sd) {
@@ -490,19 +511,19 @@ __device__ __forceinline__ void level_dispatch(int nr, const Job &J, const Team<
                                                const double2 *bv, const double2 *A, double2 *G, const double2 *g, Acc<D> &acc) {
     switch (nr) {
         case 1:
-            level_straight<D, FUSED, WAVE, L, 1>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
+            level_straight<D, FUSED, WAVE, L, 1, RM == 1>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
             break;
         case 2:
-            if constexpr (RM >= 2) level_straight<D, FUSED, WAVE, L, 2>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
+            if constexpr (RM >= 2) level_straight<D, FUSED, WAVE, L, 2, RM == 1>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
             break;
         case 3:
-            if constexpr (RM >= 3) level_straight<D, FUSED, WAVE, L, 3>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
+            if constexpr (RM >= 3) level_straight<D, FUSED, WAVE, L, 3, RM == 1>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
             break;
         case 4:
-            if constexpr (RM >= 4) level_straight<D, FUSED, WAVE, L, 4>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
+            if constexpr (RM >= 4) level_straight<D, FUSED, WAVE, L, 4, RM == 1>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
             break;
         case 5:
-            if constexpr (RM >= 5) level_straight<D, FUSED, WAVE, L, 5>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
+            if constexpr (RM >= 5) level_straight<D, FUSED, WAVE, L, 5, RM == 1>(J, tm, rank, tsize, smode, ring, kv, sq, rsq, bv, A, G, g, acc);
             break;
         default:
             break;
@@ -594,7 +615,9 @@ __device__ __forceinline__ void sweep_lds(const Bases P, const Tables T, char *l
     if (tm.rank == 0) bv[D] = P.c[J.c_off];
     const int lda = J.lda > 0 ? J.lda : D;
     for (int t = tm.rank; t < D * D; t += tm.size) am[t] = Ag[(t / D) * lda + t % D];
-    const int nrows = coef_rows(D, top);
+    constexpr bool STRAIGHT_OK = D <= 3;
+    const bool straight = STRAIGHT_OK && regp;
+    const int nrows = RM == 1 && straight ? 0 : coef_rows(D, top);  // the straight path's coefficients are in registers
     for (int t = tm.rank; t < nrows * smax; t += tm.size) {
         int r = t / smax, k = t - r * smax;
         int i = top, rr = r;
@@ -632,8 +655,6 @@ __device__ __forceinline__ void sweep_lds(const Bases P, const Tables T, char *l
     MM_PHASE(1);
 
     // straight-line path: D <= 3, whole triple in LDS, level 0 in registers
-    constexpr bool STRAIGHT_OK = D <= 3;
-    const bool straight = STRAIGHT_OK && regp;
     if (straight) {
         if constexpr (STRAIGHT_OK) {
             if constexpr (D >= 3) face_level<D, FUSED, WAVE, 2, RM>(J, tm, ring, kv, sq, rsq, bv, A, G, acc);
@@ -710,7 +731,10 @@ __device__ __forceinline__ void sweep_lds(const Bases P, const Tables T, char *l
     if (straight) {
         if constexpr (STRAIGHT_OK) {
             const int nr = (S + tm.size - 1) / tm.size;
-            level_dispatch<D, FUSED, WAVE, 0, RM>(nr, J, tm, tm.rank, tm.size, 2, ring, kv, sq, rsq, bv, A, G, g, acc);
+            if (RM == 1 && !FUSED && !WAVE && tm.size == MM_WAVE)  // a workgroup of one wave: lane moves, no barrier
+                level_straight<D, FUSED, WAVE, 0, 1, true>(J, tm, tm.rank, tm.size, 1, ring, kv, sq, rsq, bv, A, G, g, acc);
+            else
+                level_dispatch<D, FUSED, WAVE, 0, RM>(nr, J, tm, tm.rank, tm.size, 2, ring, kv, sq, rsq, bv, A, G, g, acc);
         }
     } else if (regp) {
         level0_reg<D, FUSED, WAVE, RM>(J, tm, ring, kv, sq, rsq, bv, A, G, g, coef, acc);
