@@ -366,13 +366,21 @@ Bases bases(const double *A, const double *b, const double *c, const double *g, 
 
 // --------------------------------------------------------------- slab path
 
+// One slab: fwd_slab32_kernel where its offsets and table fit.
 int launch_slab(const SlabArgs &a, int D, int64_t Sd, int num_cu, hipStream_t s) {
     int64_t blocks = (Sd + 255) / 256;
     int64_t cap = int64_t(num_cu) * 16;
     int grid = int(std::max<int64_t>(1, std::min(blocks, cap)));
+    int smax = 1;
+    for (int j = a.d + 1; j < D; ++j) smax = std::max(smax, int(a.g.shape[j]));
+    const int64_t tab = int64_t(D - 1 - a.d) * smax * 16;
+    const bool small = Sd <= SLAB32_POINTS && tab <= SLAB32_TABLE;
     switch (D) {
-#define CASE(DD) \
-    case DD: hipLaunchKernelGGL((fwd_slab_kernel<DD>), dim3(grid), dim3(256), 0, s, a); break;
+#define CASE(DD)                                                                                                              \
+    case DD:                                                                                                                  \
+        if (small) hipLaunchKernelGGL((fwd_slab32_kernel<DD>), dim3(grid), dim3(256), size_t(tab), s, a, smax);               \
+        else hipLaunchKernelGGL((fwd_slab_kernel<DD>), dim3(grid), dim3(256), 0, s, a);                                       \
+        break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
         default:
