@@ -657,10 +657,13 @@ size_t vjp_ws_bytes(const Shape &S, int64_t B) {
 template <int D, bool SLAB, bool FWD>
 void launch_vjp_kernel_t(const VjpArgs &a, int64_t B, hipStream_t s) {
     const dim3 grid(unsigned(a.nchunk * RowSplit<D>::NG), unsigned(B));
-    if (a.smax <= VJP_LDS_SQ)
-        hipLaunchKernelGGL((vjp_kernel<D, SLAB, FWD, true>), grid, dim3(256), size_t(a.smax + 2) * 8, s, a);
+    const bool small = (SLAB ? a.g.stride[0] : a.g.N) <= SLAB32_POINTS;
+    if (a.smax > VJP_LDS_SQ)
+        hipLaunchKernelGGL((vjp_kernel<D, SLAB, FWD, false, false>), grid, dim3(256), 0, s, a);
+    else if (small)
+        hipLaunchKernelGGL((vjp_kernel<D, SLAB, FWD, true, true>), grid, dim3(256), size_t(a.smax + 2) * 8, s, a);
     else
-        hipLaunchKernelGGL((vjp_kernel<D, SLAB, FWD, false>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((vjp_kernel<D, SLAB, FWD, true, false>), grid, dim3(256), size_t(a.smax + 2) * 8, s, a);
 }
 
 int launch_finalize(int D, int64_t B, const double2 *partial, int nchunk, const double *c, double *dA, double *db, double *dc, bool conj,

@@ -15,6 +15,8 @@
 // deterministic.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "exact.hpp"
 #include "global_kernels.hpp"
@@ -103,26 +105,35 @@ struct RowSplit {
 // of one XCD (blk % 8, see xcd_block) take neighbouring visits and all
 // blocks advance through the lattice together, so the strided neighbours of a
 // point were or will be read nearby in time.
-template <int D, int R0, int R1, bool SLAB, bool FWD, bool LT>
+template <int D, int R0, int R1, bool SLAB, bool FWD, bool LT, bool I32>
 __device__ __forceinline__ void vjp_group(const VjpArgs &a, const double *sqt, int blk, double2 *row) {
     using RG = RowGroup<D, R0, R1>;
     constexpr int NL = RG::NL;
     constexpr int LO = SLAB ? 1 : 0;  // first axis with a digit
     const double *sq = LT ? sqt : a.sq;
-    const int64_t S = SLAB ? a.g.stride[0] : a.g.N;
+    // I32: the points' byte offsets from the arrays' (uniform) addresses fit 32
+    // bits.  Half of the kernel's issue slots were busy, a third of them with 64-bit
+    // addresses: a slab of 10^7 points of D = 8 with the next one formed 367 -> 322 us
+    // (1.1 GB, 3.5 TB/s), (12,)^6 52.5 -> 48.
+    using X = std::conditional_t<I32, uint32_t, int64_t>;
+    auto at = [](const double2 *p, X x) {
+        if constexpr (I32) return *reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(p) + x * 16u);
+        else return p[x];
+    };
+    const X S = X(SLAB ? a.g.stride[0] : a.g.N);
     double2 acc[NL];
 #pragma unroll
     for (int e = 0; e < NL; ++e) acc[e] = make_double2(0.0, 0.0);
     const int m = a.m;
-    const int64_t round = int64_t(a.nchunk) * 256 * a.visit;
+    const X round = X(a.nchunk) * 256 * a.visit;
     const int place = a.nchunk % MM_XCDS == 0 ? (blk % MM_XCDS) * (a.nchunk / MM_XCDS) + blk / MM_XCDS : blk;
-    int64_t q = int64_t(place) * 256 * a.visit + threadIdx.x;
-    const int64_t hop = round - int64_t(256) * (a.visit - 1);
-    int64_t stl[D];
+    X q = X(place) * 256 * a.visit + threadIdx.x;
+    const X hop = round - X(256) * (a.visit - 1);
+    X stl[D];
     int k[D], kin[D], khop[D];
 #pragma unroll
     for (int i = 0; i < D; ++i) {
-        stl[i] = a.g.stride[i];
+        stl[i] = X(a.g.stride[i]);
         k[i] = kin[i] = khop[i] = 0;
     }
     if (q < S) {
@@ -145,27 +156,27 @@ __device__ __forceinline__ void vjp_group(const VjpArgs &a, const double *sqt, i
     int it = 0;
     while (q < S) {
         // every load of the point first: one round trip
-        const double2 G0 = a.G[q];
-        const double2 g0 = R0 == 0 ? a.gg[q] : make_double2(0.0, 0.0);
+        const double2 G0 = at(a.G, q);
+        const double2 g0 = R0 == 0 ? at(a.gg, q) : make_double2(0.0, 0.0);
         double2 v[D], u[D];
         double wd[D], wu[D];
 #pragma unroll
         for (int j = 0; j < D; ++j) {
             if (j < R0) continue;
             if (SLAB && j == 0) {
-                v[0] = a.Gdn[q];
+                v[0] = at(a.Gdn, q);
                 wd[0] = wdn0;
             } else {
-                v[j] = a.G[q - (k[j] > 0 ? stl[j] : 0)];
+                v[j] = at(a.G, q - (k[j] > 0 ? stl[j] : 0));
                 wd[j] = sq[k[j]];
             }
             if (j >= R1) continue;
             if (SLAB && j == 0) {
-                u[0] = a.gup[q];
+                u[0] = at(a.gup, q);
                 wu[0] = wup0;
             } else {
                 const bool up = k[j] + 1 < a.g.shape[j];
-                u[j] = a.gg[q + (up ? stl[j] : 0)];
+                u[j] = at(a.gg, q + (up ? stl[j] : 0));
                 const double w = sq[k[j] + 1];
                 wu[j] = up ? w : 0.0;
             }
@@ -176,7 +187,8 @@ __device__ __forceinline__ void vjp_group(const VjpArgs &a, const double *sqt, i
             if (m >= 1) o = cadd(o, cmul(c00, v[0]));
 #pragma unroll
             for (int j = 1; j < D; ++j) o = cadd(o, cmul(cscale_promoted(A0[j], wd[j]), v[j]));
-            a.nxt[q] = cdiv_by(o, sm, rm);
+            if constexpr (I32) *reinterpret_cast<double2 *>(reinterpret_cast<char *>(a.nxt) + q * 16u) = cdiv_by(o, sm, rm);
+            else a.nxt[q] = cdiv_by(o, sm, rm);
         }
         if (R0 == 0) acc[RG::lc()] = cfma(G0, make_double2(g0.x, gs * g0.y), acc[RG::lc()]);
 #pragma unroll
@@ -208,7 +220,7 @@ __device__ __forceinline__ void vjp_group(const VjpArgs &a, const double *sqt, i
     block_store_group<D, R0, R1>(acc, row, SLAB && m > 0);
 }
 
-template <int D, bool SLAB, bool FWD, bool LT>
+template <int D, bool SLAB, bool FWD, bool LT, bool I32>
 __global__ __launch_bounds__(256, D <= 4 ? 3 : 2) void vjp_kernel(VjpArgs a) {
     extern __shared__ double sqt[];
     using RS = RowSplit<D>;
@@ -234,9 +246,9 @@ __global__ __launch_bounds__(256, D <= 4 ? 3 : 2) void vjp_kernel(VjpArgs a) {
     }
     double2 *row = a.partial + (t * a.nchunk + blk) * NA;
     if (grp == 0) {
-        vjp_group<D, 0, RS::B1, SLAB, FWD, LT>(a, sqt, blk, row);
+        vjp_group<D, 0, RS::B1, SLAB, FWD, LT, I32>(a, sqt, blk, row);
     } else {
-        if constexpr (RS::NG == 2) vjp_group<D, RS::B1, D, SLAB, false, LT>(a, sqt, blk, row);
+        if constexpr (RS::NG == 2) vjp_group<D, RS::B1, D, SLAB, false, LT, I32>(a, sqt, blk, row);
     }
 }
 
