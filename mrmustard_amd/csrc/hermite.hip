@@ -975,7 +975,7 @@ int vanilla_uniform(const Shape &S, int64_t B, const double *A, const double *b,
         sa.nf = nf;
         // with the VJP of a single triple above 512 MB, each level-0 launch
         // takes the VJP terms of slab m and the forward of slab m + 1 from the
-        // same loads; below that, the forward (two slabs per launch) then one
+        // same loads; below that, the forward (several slabs per launch) then one
         // VJP pass take fewer launches
         const bool fuse_level0 = fused && B == 1 && S.N * 16 > (int64_t(512) << 20);
         for (int d = top - 1; d >= (fuse_level0 ? 1 : 0); --d) {

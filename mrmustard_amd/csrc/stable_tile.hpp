@@ -17,8 +17,8 @@
 // The rows are dealt to the lanes by digit sum, so that a wave without a point
 // in a step skips it.  Every term, order and rounding is that of stable_point.
 // Measured, one launch per index sum (or one workgroup per triple) against the
-// tiles: (40,)^4 858 -> 550 us (25 launches of 5 x 5 x 5 x 10 tiles, 22 steps of
-// ~0.5 us each), (70, 70, 60) 752 -> 344 us, (1000, 1000) 6529 -> 1970 us (31
+// tiles: (40,)^4 858 -> 550 us (37 launches of 4^4 tiles, 13 steps of ~0.5 us
+// each), (70, 70, 60) 752 -> 344 us, (1000, 1000) 6529 -> 1970 us (31
 // launches), (20,)^5 1206 -> 906 us, (50, 50) 100 -> 41 us (the whole lattice one
 // tile), 1000 of (5,)^4 142 -> 43 us; but (11,)^6 912 -> 1521 us, where the halo of
 // a 2^6 tile is ten times its points: the caller compares both estimates.
