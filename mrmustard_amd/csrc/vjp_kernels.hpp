@@ -10,9 +10,9 @@
 // so a point gathers 2 D + 2 values instead of one per sum (D (D + 3) / 2 + 2)
 // and no cotangent twice.  A zero weight (q_j = 0, or q_i the last of its
 // axis) reads the point itself: branch-free, all gathers issue together.
-// The sums live in registers, a block reduces them with DPP moves and LDS and
-// writes one partial row, vjp_finalize adds the rows of a triple in order:
-// deterministic.
+// The sums live in registers, a wave takes them over every VJP_CHAIN points
+// (one sum per lane), a block adds its waves' and writes one partial row,
+// vjp_finalize adds the rows of a triple in order: deterministic.
 #pragma once
 
 #include <type_traits>
@@ -26,6 +26,15 @@ namespace mm {
 // Largest axis whose square roots sit in LDS (LT kernels); longer ones are
 // read from the device table.
 constexpr int VJP_LDS_SQ = 4096;
+
+// Points that a thread sums before the wave takes its sums: the rounding error
+// of a chain of n terms grows as sqrt(n), and large lattices have hundreds of
+// points per thread.  Error of the sums in eps sqrt(sum |term|^2), chains of
+// all points against these: (11,)^7 kets 4.7 -> 1.3, (8,)^8 density matrices 3.4
+// -> 1.3, (10,)^8 slab by slab 3.3 -> 1.2, (12,)^6 1.7 -> 1.1; the time of all of
+// them is the same within 1 % (a scatter_sum is 5 to 7 % of 16 points' instructions,
+// and the kernel waits for memory).
+constexpr int VJP_CHAIN = 16;
 
 struct VjpArgs {
     Geom g;
@@ -68,25 +77,76 @@ struct RowGroup {
     }
 };
 
-// Reduce NL sums over the block (DPP within waves, waves in order) and store
-// them in, or add them to, the block's partial row at the group's columns.
-template <int D, int R0, int R1, int NL>
-__device__ __forceinline__ void block_store_group(double2 (&acc)[NL], double2 *row, bool add) {
-    using RG = RowGroup<D, R0, R1>;
-    static_assert(NL == RG::NL, "accumulator count");
-    __shared__ double2 red[(256 / MM_WAVE) * NL];
-    wave_sum_dpp<NL>(acc);
-    const int lane = threadIdx.x & (MM_WAVE - 1), w = threadIdx.x / MM_WAVE;
-    if (lane == MM_WAVE - 1) {
-#pragma unroll
-        for (int e = 0; e < NL; ++e) red[w * NL + e] = acc[e];
+// Sums of N <= 64 values over the wave, lane l keeping the sum of value
+// bit-reverse(l) (6 bits): each stage halves the values instead of summing all
+// of them on every lane, 240 instructions for 60 values where wave_sum_dpp has
+// 1,080.  The order is fixed.
+template <int STAGE>
+__device__ __forceinline__ double pair_sum(double x, double y) {
+    if constexpr (STAGE < 2) {
+        // lanes 32 (16) and up of x against those below of y
+        auto swap = [](int u, int v) {
+            if constexpr (STAGE == 0) return __builtin_amdgcn_permlane32_swap(u, v, false, false);
+            else return __builtin_amdgcn_permlane16_swap(u, v, false, false);
+        };
+        const auto lo = swap(__double2loint(x), __double2loint(y));
+        const auto hi = swap(__double2hiint(x), __double2hiint(y));
+        return __hiloint2double(int(hi[0]), int(lo[0])) + __hiloint2double(int(hi[1]), int(lo[1]));
+    } else {
+        // row_mirror, row_half_mirror, quad_perm [2,3,0,1] and [1,0,3,2]
+        constexpr int CTRL[] = {0x140, 0x141, 0x4E, 0xB1};
+        const bool up = (threadIdx.x >> (5 - STAGE)) & 1;
+        const double keep = up ? y : x, give = up ? x : y;
+        return keep + dpp_d<CTRL[STAGE - 2], 0xF>(give);
     }
+}
+
+template <int STAGE, int N>
+__device__ __forceinline__ double scatter_sum(const double (&v)[N]) {
+    constexpr int H = (N + 1) / 2;
+    double h[H];
+#pragma unroll
+    for (int i = 0; i < H; ++i) h[i] = pair_sum<STAGE>(v[2 * i], 2 * i + 1 < N ? v[2 * i + 1] : 0.0);
+    if constexpr (STAGE == 5) return h[0];
+    else return scatter_sum<STAGE + 1>(h);
+}
+
+// Move a thread's sums into the lane's own one of the wave (component 2 l of
+// sum l, 2 l + 1 its imaginary part), and start them again from zero.
+template <int D, int R0, int R1, int NL>
+__device__ __forceinline__ void flush_sums(double2 (&acc)[NL], double &held) {
+    using RG = RowGroup<D, R0, R1>;
+    static_assert(NL == RG::NL && 2 * NL <= MM_WAVE, "accumulator count");
+    double v[2 * NL];
+#pragma unroll
+    for (int e = 0; e < NL; ++e) {
+        v[2 * e] = acc[e].x;
+        v[2 * e + 1] = acc[e].y;
+        acc[e] = make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int i = R0; i < R1; ++i) {  // dA_ii = sum u_i v_i / 2
+        v[2 * RG::la(i, i)] *= 0.5;
+        v[2 * RG::la(i, i) + 1] *= 0.5;
+    }
+    held += scatter_sum<0>(v);
+}
+
+// Sum the waves' held sums in order and store them in, or add them to, the
+// block's partial row at the group's columns.
+template <int D, int R0, int R1>
+__device__ __forceinline__ void block_store_group(double held, double2 *row, bool add) {
+    using RG = RowGroup<D, R0, R1>;
+    __shared__ double red[256];
+    red[threadIdx.x] = held;
     __syncthreads();
-    if (threadIdx.x < NL) {
-        double2 t = red[threadIdx.x];
-        for (int ww = 1; ww < int(blockDim.x / MM_WAVE); ++ww) t = cadd(t, red[ww * NL + threadIdx.x]);
-        const int col = RG::column(threadIdx.x);
-        row[col] = add ? cadd(row[col], t) : t;
+    const int t = threadIdx.x;
+    if (t < 2 * RG::NL) {
+        const int lane = int(__brev(uint32_t(t)) >> 26);
+        double sum = red[lane];
+        for (int w = 1; w < 256 / MM_WAVE; ++w) sum += red[w * MM_WAVE + lane];
+        double *out = reinterpret_cast<double *>(row + RG::column(t / 2)) + (t & 1);
+        *out = add ? *out + sum : sum;
     }
 }
 
@@ -127,7 +187,9 @@ __device__ __forceinline__ void vjp_group(const VjpArgs &a, const double *sqt, i
     const int m = a.m;
     const X round = X(a.nchunk) * 256 * a.visit;
     const int place = a.nchunk % MM_XCDS == 0 ? (blk % MM_XCDS) * (a.nchunk / MM_XCDS) + blk / MM_XCDS : blk;
-    X q = X(place) * 256 * a.visit + threadIdx.x;
+    // points are taken from the last one down, q = S - 1 - p: the amplitudes of
+    // a state fall off with the photon numbers, and small terms go first
+    X p = X(place) * 256 * a.visit;  // of thread 0
     const X hop = round - X(256) * (a.visit - 1);
     X stl[D];
     int k[D], kin[D], khop[D];
@@ -136,10 +198,11 @@ __device__ __forceinline__ void vjp_group(const VjpArgs &a, const double *sqt, i
         stl[i] = X(a.g.stride[i]);
         k[i] = kin[i] = khop[i] = 0;
     }
-    if (q < S) {
-        digits_of<D>(q, a.g, LO, k);
-        digits_of<D>(256 < S ? 256 : 0, a.g, LO, kin);
-        digits_of<D>(hop < S ? hop : 0, a.g, LO, khop);
+    if (p + threadIdx.x < S) {
+        // a step down is one up by S less, its last carry dropped
+        digits_of<D>(S - 1 - (p + threadIdx.x), a.g, LO, k);
+        digits_of<D>(256 < S ? S - 256 : 0, a.g, LO, kin);
+        digits_of<D>(hop < S ? S - hop : 0, a.g, LO, khop);
     }
     const double gs = a.gsign;
     const double wdn0 = a.sq[m], wup0 = m + 1 < a.g.shape[0] ? a.sq[m + 1] : 0.0;  // SLAB: axis 0
@@ -153,71 +216,75 @@ __device__ __forceinline__ void vjp_group(const VjpArgs &a, const double *sqt, i
 #pragma unroll
         for (int j = 0; j < D; ++j) A0[j] = a.A[j];
     }
-    int it = 0;
-    while (q < S) {
-        // every load of the point first: one round trip
-        const double2 G0 = at(a.G, q);
-        const double2 g0 = R0 == 0 ? at(a.gg, q) : make_double2(0.0, 0.0);
-        double2 v[D], u[D];
-        double wd[D], wu[D];
+    int it = 0, chain = 0;
+    double held = 0.0;
+    while (p < S) {
+        if (p + threadIdx.x < S) {
+            const X q = S - 1 - (p + threadIdx.x);
+            // every load of the point first: one round trip
+            const double2 G0 = at(a.G, q);
+            const double2 g0 = R0 == 0 ? at(a.gg, q) : make_double2(0.0, 0.0);
+            double2 v[D], u[D];
+            double wd[D], wu[D];
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-            if (j < R0) continue;
-            if (SLAB && j == 0) {
-                v[0] = at(a.Gdn, q);
-                wd[0] = wdn0;
-            } else {
-                v[j] = at(a.G, q - (k[j] > 0 ? stl[j] : 0));
-                wd[j] = sq[k[j]];
+            for (int j = 0; j < D; ++j) {
+                if (j < R0) continue;
+                if (SLAB && j == 0) {
+                    v[0] = at(a.Gdn, q);
+                    wd[0] = wdn0;
+                } else {
+                    v[j] = at(a.G, q - (k[j] > 0 ? stl[j] : 0));
+                    wd[j] = sq[k[j]];
+                }
+                if (j >= R1) continue;
+                if (SLAB && j == 0) {
+                    u[0] = at(a.gup, q);
+                    wu[0] = wup0;
+                } else {
+                    const bool up = k[j] + 1 < a.g.shape[j];
+                    u[j] = at(a.gg, q + (up ? stl[j] : 0));
+                    const double w = sq[k[j] + 1];
+                    wu[j] = up ? w : 0.0;
+                }
             }
-            if (j >= R1) continue;
-            if (SLAB && j == 0) {
-                u[0] = at(a.gup, q);
-                wu[0] = wup0;
-            } else {
-                const bool up = k[j] + 1 < a.g.shape[j];
-                u[j] = at(a.gg, q + (up ? stl[j] : 0));
-                const double w = sq[k[j] + 1];
-                wu[j] = up ? w : 0.0;
+            if (FWD) {
+                // the recurrence of fwd_slab0_kernel for slab m + 1, same order of operations
+                double2 o = cmul(b0, G0);
+                if (m >= 1) o = cadd(o, cmul(c00, v[0]));
+#pragma unroll
+                for (int j = 1; j < D; ++j) o = cadd(o, cmul(cscale_promoted(A0[j], wd[j]), v[j]));
+                if constexpr (I32) *reinterpret_cast<double2 *>(reinterpret_cast<char *>(a.nxt) + q * 16u) = cdiv_by(o, sm, rm);
+                else a.nxt[q] = cdiv_by(o, sm, rm);
+            }
+            if (R0 == 0) acc[RG::lc()] = cfma(G0, make_double2(g0.x, gs * g0.y), acc[RG::lc()]);
+#pragma unroll
+            for (int j = 0; j < D; ++j) {
+                if (j < R0) continue;
+                v[j] = make_double2(wd[j] * v[j].x, wd[j] * v[j].y);
+            }
+#pragma unroll
+            for (int i = R0; i < R1; ++i) {
+                const double2 ui = make_double2(wu[i] * u[i].x, (wu[i] * gs) * u[i].y);
+                acc[RG::lb(i)] = cfma(G0, ui, acc[RG::lb(i)]);
+#pragma unroll
+                for (int j = i; j < D; ++j) acc[RG::la(i, j)] = cfma(v[j], ui, acc[RG::la(i, j)]);
             }
         }
-        if (FWD) {
-            // the recurrence of fwd_slab0_kernel for slab m + 1, same order of operations
-            double2 o = cmul(b0, G0);
-            if (m >= 1) o = cadd(o, cmul(c00, v[0]));
-#pragma unroll
-            for (int j = 1; j < D; ++j) o = cadd(o, cmul(cscale_promoted(A0[j], wd[j]), v[j]));
-            if constexpr (I32) *reinterpret_cast<double2 *>(reinterpret_cast<char *>(a.nxt) + q * 16u) = cdiv_by(o, sm, rm);
-            else a.nxt[q] = cdiv_by(o, sm, rm);
-        }
-        if (R0 == 0) acc[RG::lc()] = cfma(G0, make_double2(g0.x, gs * g0.y), acc[RG::lc()]);
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-            if (j < R0) continue;
-            v[j] = make_double2(wd[j] * v[j].x, wd[j] * v[j].y);
-        }
-#pragma unroll
-        for (int i = R0; i < R1; ++i) {
-            const double2 ui = make_double2(wu[i] * u[i].x, (wu[i] * gs) * u[i].y);
-            acc[RG::lb(i)] = cfma(G0, ui, acc[RG::lb(i)]);
-#pragma unroll
-            for (int j = i; j < D; ++j) acc[RG::la(i, j)] = cfma(v[j], ui, acc[RG::la(i, j)]);
+        if (++chain == VJP_CHAIN) {
+            chain = 0;
+            flush_sums<D, R0, R1>(acc, held);
         }
         if (++it < a.visit) {
-            q += 256;
+            p += 256;
             digits_add<D>(k, kin, a.g, LO);
         } else {
             it = 0;
-            q += hop;
+            p += hop;
             digits_add<D>(k, khop, a.g, LO);
         }
     }
-#pragma unroll
-    for (int i = R0; i < R1; ++i) {
-        double2 &d = acc[RG::la(i, i)];
-        d = make_double2(0.5 * d.x, 0.5 * d.y);
-    }
-    block_store_group<D, R0, R1>(acc, row, SLAB && m > 0);
+    flush_sums<D, R0, R1>(acc, held);
+    block_store_group<D, R0, R1>(held, row, SLAB && m > 0);
 }
 
 template <int D, bool SLAB, bool FWD, bool LT, bool I32>
