@@ -304,6 +304,12 @@ int mm_zgemm(const double *A, int64_t lda, const double *B, int64_t ldb, double 
 int mm_zgemm_batched(const double *A, int64_t lda, int64_t sA, const double *B, int64_t ldb, int64_t sB, double *C, int64_t ldc,
                      int64_t sC, int64_t M, int64_t N, int64_t K, int64_t batch, void *stream);
 
+/* How mm_zgemm_batched cuts a batch into launches on num_cu compute units
+ * (host, 4 entries): 16-row tiles of a workgroup (0: 64 x 128 tiles), products
+ * of a launch, columns of each, 1 when their columns are merged into one
+ * product (shared_a: all products have the same A). */
+int mm_zgemm_plan(int64_t M, int64_t N, int64_t batch, int shared_a, int num_cu, int64_t *out);
+
 /* ------------------------------------------------- work-queue batch (plans)
  *
  * A plan describes n triples of uneven mode count D_k <= 8 and shape_k.

@@ -24,6 +24,33 @@ int strip_rt(int64_t M, int64_t N, int64_t batch, int num_cu) {
     return int((mt + gy - 1) / gy);
 }
 
+// HIP takes launches of fewer than 2^32 threads along x: 2^24 - 1 workgroups of 256.
+constexpr int64_t MAX_GX = (int64_t(1) << 24) - 1;
+
+// How a batch of products is cut into launches: `step` products of `cols`
+// columns each; merged: the columns of all of them as one product (cols = N).
+struct ZgemmPlan {
+    int rt = 0;
+    int64_t step = 0, cols = 0;
+    bool merged = false;
+};
+
+// false when one product has more columns or rows than a launch of
+// zgemm_mfma_kernel takes.
+bool zgemm_plan(int64_t M, int64_t N, int64_t batch, bool shared_a, int num_cu, ZgemmPlan *p) {
+    if (N > MAX_GX * ZG_BN || (M + 63) / 64 > 65535) return false;
+    p->rt = strip_rt(M, N, batch, num_cu);
+    p->step = std::min<int64_t>(batch, 65535);  // grid z
+    p->cols = N;
+    if (p->rt) {
+        const int64_t most = MAX_GX * 64;  // columns of a launch of zgemm_strip_kernel
+        p->merged = shared_a && batch > 1 && N <= most / 2;
+        if (p->merged) p->step = std::min<int64_t>(batch, most / N);
+        else p->cols = std::min<int64_t>(N, most);
+    }
+    return true;
+}
+
 // nz products of N columns each, or (cols > N) one with the columns of all.
 template <int RT>
 void launch_strip(const ZgemmArgs &a, int64_t nz, int64_t cols, hipStream_t s) {
@@ -50,15 +77,14 @@ int mm_zgemm_batched(const double *A, int64_t lda, int64_t sA, const double *B, 
     if (lda < K || ldb < N || ldc < N) return fail(MM_ERR_INVALID, "leading dimension smaller than the row length");
     if (sA < 0 || sB < 0 || sC < 0) return fail(MM_ERR_INVALID, "negative batch stride");
     if (batch > 1 && sC < (M - 1) * ldc + N) return fail(MM_ERR_INVALID, "the products of a batch overlap in C");
-    const int64_t gx = (N + ZG_BN - 1) / ZG_BN, gy = (M + 63) / 64;
-    if (gx > 0x3fffffff || gy > 65535) return fail(MM_ERR_UNSUPPORTED, "matrix too large for one launch");
     DevState *ds = nullptr;
     const int rc = device_state(&ds);
     if (rc) return rc;
-    const int rt = strip_rt(M, N, batch, ds->num_cu);
+    ZgemmPlan p;
+    // products that share A are merged into one with all their columns
+    if (!zgemm_plan(M, N, batch, sA == 0, ds->num_cu, &p)) return fail(MM_ERR_UNSUPPORTED, "matrix too large for one launch");
     ZgemmArgs a;
     a.M = M;
-    a.N = N;
     a.K = K;
     a.lda = lda;
     a.ldb = ldb;
@@ -67,31 +93,47 @@ int mm_zgemm_batched(const double *A, int64_t lda, int64_t sA, const double *B, 
     a.sB = sB;
     a.sC = sC;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    // products that share A: one with all their columns, while grid x holds it
-    const bool flat = rt && sA == 0 && batch > 1 && N <= (int64_t(1) << 36) / batch;
-    const int64_t step = flat ? batch : 65535;  // grid z holds at most 65535 products
-    for (int64_t b0 = 0; b0 < batch; b0 += step) {
-        const int64_t nz = std::min<int64_t>(step, batch - b0);
-        a.A = reinterpret_cast<const double2 *>(A) + b0 * sA;
-        a.B = reinterpret_cast<const double2 *>(B) + b0 * sB;
-        a.C = reinterpret_cast<double2 *>(C) + b0 * sC;
-        switch (rt) {
-            case 0:
-                hipLaunchKernelGGL(zgemm_mfma_kernel, dim3(unsigned(gx), unsigned(gy), unsigned(nz)), dim3(256), 0, s, a);
-                break;
-#define CASE(RT) \
-    case RT: launch_strip<RT>(a, flat ? 1 : nz, flat ? N * nz : N, s); break;
-                CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+    for (int64_t b0 = 0; b0 < batch; b0 += p.step)
+        for (int64_t n0 = 0; n0 < N; n0 += p.cols) {
+            const int64_t nz = std::min<int64_t>(p.step, batch - b0);
+            a.N = std::min<int64_t>(p.cols, N - n0);
+            a.A = reinterpret_cast<const double2 *>(A) + b0 * sA;
+            a.B = reinterpret_cast<const double2 *>(B) + b0 * sB + n0;
+            a.C = reinterpret_cast<double2 *>(C) + b0 * sC + n0;
+            switch (p.rt) {
+                case 0: {
+                    const dim3 grid(unsigned((N + ZG_BN - 1) / ZG_BN), unsigned((M + 63) / 64), unsigned(nz));
+                    hipLaunchKernelGGL(zgemm_mfma_kernel, grid, dim3(256), 0, s, a);
+                    LAUNCH_CHECK("zgemm_mfma_kernel");
+                    break;
+                }
+#define CASE(RT)                                                                    \
+    case RT:                                                                        \
+        launch_strip<RT>(a, p.merged ? 1 : nz, p.merged ? N * nz : a.N, s);         \
+        LAUNCH_CHECK("zgemm_strip_kernel");                                         \
+        break;
+                    CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
+            }
         }
-    }
-    LAUNCH_CHECK("zgemm_mfma_kernel");
     return MM_OK;
 }
 
 int mm_zgemm(const double *A, int64_t lda, const double *B, int64_t ldb, double *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
              void *stream) {
     return mm_zgemm_batched(A, lda, 0, B, ldb, 0, C, ldc, 0, M, N, K, 1, stream);
+}
+
+int mm_zgemm_plan(int64_t M, int64_t N, int64_t batch, int shared_a, int num_cu, int64_t *out) {
+    if (!out) return fail(MM_ERR_INVALID, "NULL pointer");
+    if (M < 1 || N < 1 || batch < 1 || num_cu < 1) return fail(MM_ERR_INVALID, "sizes must be positive");
+    ZgemmPlan p;
+    if (!zgemm_plan(M, N, batch, shared_a != 0, num_cu, &p)) return fail(MM_ERR_UNSUPPORTED, "matrix too large for one launch");
+    out[0] = p.rt;
+    out[1] = p.step;
+    out[2] = p.cols;
+    out[3] = p.merged;
+    return MM_OK;
 }
 
 }  // extern "C"
