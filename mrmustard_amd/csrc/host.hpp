@@ -80,6 +80,15 @@ inline int device_state(DevState **out) {
     return MM_OK;
 }
 
+// Compute units of the current device, without the tables of device_state:
+// no allocation, so also inside a stream capture.
+inline int compute_units(int *out) {
+    int dev = 0;
+    HIP_TRY(hipGetDevice(&dev));
+    HIP_TRY(hipDeviceGetAttribute(out, hipDeviceAttributeMultiprocessorCount, dev));
+    return MM_OK;
+}
+
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 }  // namespace mm

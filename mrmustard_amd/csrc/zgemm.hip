@@ -77,12 +77,12 @@ int mm_zgemm_batched(const double *A, int64_t lda, int64_t sA, const double *B, 
     if (lda < K || ldb < N || ldc < N) return fail(MM_ERR_INVALID, "leading dimension smaller than the row length");
     if (sA < 0 || sB < 0 || sC < 0) return fail(MM_ERR_INVALID, "negative batch stride");
     if (batch > 1 && sC < (M - 1) * ldc + N) return fail(MM_ERR_INVALID, "the products of a batch overlap in C");
-    DevState *ds = nullptr;
-    const int rc = device_state(&ds);
+    int num_cu = 1;
+    const int rc = compute_units(&num_cu);
     if (rc) return rc;
     ZgemmPlan p;
     // products that share A are merged into one with all their columns
-    if (!zgemm_plan(M, N, batch, sA == 0, ds->num_cu, &p)) return fail(MM_ERR_UNSUPPORTED, "matrix too large for one launch");
+    if (!zgemm_plan(M, N, batch, sA == 0, num_cu, &p)) return fail(MM_ERR_UNSUPPORTED, "matrix too large for one launch");
     ZgemmArgs a;
     a.M = M;
     a.K = K;
