@@ -157,6 +157,9 @@ def leftover_grad_hip(A, b, c, output_cutoff: int, pnr_cutoffs, ws, grad, reorde
     reverse sweep of ``leftover_vjp_hip`` without a second forward."""
     A, b, c, g = as_device_c128(A), as_device_c128(b), as_device_c128(c), as_device_c128(grad)
     pnr = tuple(int(k) for k in pnr_cutoffs)
+    M = len(pnr) + 1
+    if tuple(A.shape) != (2 * M, 2 * M) or tuple(b.shape) != (2 * M,) or c.numel() != 1:
+        raise ValueError(f"A must be ({2 * M}, {2 * M}), b ({2 * M},) and c scalar for {M} modes")
     o = int(output_cutoff)
     if tuple(g.shape) != (o + 1, o + 1, *(k + 1 for k in pnr)):
         raise ValueError("the gradient must have the shape of the output")
