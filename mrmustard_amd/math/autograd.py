@@ -19,6 +19,7 @@ from __future__ import annotations
 import torch
 
 from ..lattice import strategies as st
+from ..settings import settings
 
 
 class HermiteRenormalized(torch.autograd.Function):
@@ -115,15 +116,15 @@ class HermiteLeftover(torch.autograd.Function):
     pair, jax_vjps/hermite.py:343-445).  The forward's intermediate blocks are
     kept for the backward up to ``LEFTOVER_KEEP_BYTES`` (a (20, 20, 15, 15)
     output: 16 MB; its second forward took a quarter of a training step);
-    beyond that only (A, b, c) are kept and the backward recomputes them
-    (``leftover_vjp_hip``)."""
+    beyond that, or with ``settings.HERMITE_RECOMPUTE_VJP``, only (A, b, c) are
+    kept and the backward recomputes them (``leftover_vjp_hip``)."""
 
     @staticmethod
     def forward(ctx, A, b, c, output_cutoff, pnr_cutoffs, reordered):
         from ..lattice import compact_fock as cf
 
         out, ws = cf._leftover(A, b, c, output_cutoff, pnr_cutoffs, reordered)
-        if ws.numel() <= cf.LEFTOVER_KEEP_BYTES:
+        if ws.numel() <= cf.LEFTOVER_KEEP_BYTES and not settings.HERMITE_RECOMPUTE_VJP:
             ctx.save_for_backward(A, b, c, ws)
         else:
             ctx.save_for_backward(A, b, c)

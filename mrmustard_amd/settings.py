@@ -23,7 +23,8 @@ class Settings:
             # settings.py:101 -- ORed into `stable` by backend_manager.py:682
             inst.STABLE_FOCK_CONVERSION = False
             # not in the reference: autograd keeps only (A, b, c) and the backward
-            # recomputes the lattice slab by slab (bounded memory)
+            # recomputes the lattice slab by slab, or the leftover-mode strategy's
+            # blocks (bounded memory)
             inst.HERMITE_RECOMPUTE_VJP = False
             # settings.py:79, :67-74 (consumed by callers that pick a shape)
             inst.DEFAULT_FOCK_SIZE = 50
