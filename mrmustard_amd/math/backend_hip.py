@@ -67,8 +67,7 @@ class BackendHip:
 
     def reshape(self, array, shape):
         if isinstance(array, torch.Tensor):
-            # no view (and no node of one) where there is nothing to reshape
-            return array if array.shape == tuple(shape) else array.reshape(tuple(shape))
+            return array.reshape(tuple(shape))
         return np.reshape(array, tuple(shape))
 
     def broadcast_to(self, array, shape):

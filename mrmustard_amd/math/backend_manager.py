@@ -22,6 +22,7 @@ from math import prod
 from typing import Any
 
 import numpy as np
+import torch
 
 from ..settings import settings
 from .backend_hip import BackendHip
@@ -127,28 +128,28 @@ class BackendManager:
             if tuple(c.shape[: len(batch_shape)]) != batch_shape:
                 raise ValueError(f"c.shape={tuple(c.shape)} must match batch_shape={batch_shape}")
             D = prod(batch_shape)
-            A = self.reshape(A, (D, *A.shape[-2:]))
-            b = self.reshape(b, (D, *b.shape[-1:]))
-            c = self.reshape(c, (D,))
+            A = self._shaped(A, (D, *A.shape[-2:]))
+            b = self._shaped(b, (D, *b.shape[-1:]))
+            c = self._shaped(c, (D,))
             result = self._apply(
                 "hermite_renormalized_batched",
                 (A, b, c),
-                {"shape": tuple(shape), "stable": stable, "out": self.reshape(out, (D, *shape)) if out is not None else None},
+                {"shape": tuple(shape), "stable": stable, "out": self._shaped(out, (D, *shape)) if out is not None else None},
             )
-            return self.reshape(result, batch_shape + tuple(shape))
+            return self._shaped(result, batch_shape + tuple(shape))
         if A.ndim == 2 and b.ndim > 1:  # b-batched case
             batch_shape = tuple(b.shape[:-1])
             check_out_shape(batch_shape)
             D = prod(batch_shape)
-            b = self.reshape(b, (D, *b.shape[-1:]))
+            b = self._shaped(b, (D, *b.shape[-1:]))
             A_broadcast = self.broadcast_to(A, (D, *A.shape))
             c_broadcast = self.broadcast_to(c, (D,))
             result = self._apply(
                 "hermite_renormalized_batched",
                 (A_broadcast, b, c_broadcast),
-                {"shape": tuple(shape), "stable": stable, "out": self.reshape(out, (D, *shape)) if out is not None else None},
+                {"shape": tuple(shape), "stable": stable, "out": self._shaped(out, (D, *shape)) if out is not None else None},
             )
-            return self.reshape(result, batch_shape + tuple(shape))
+            return self._shaped(result, batch_shape + tuple(shape))
         check_out_shape(())
         return self._apply("hermite_renormalized", (A, b, c), {"shape": tuple(shape), "stable": stable, "out": out})
 
@@ -185,6 +186,11 @@ class BackendManager:
         from ..contraction import einsum as _einsum
 
         return _einsum(string, *tensors)
+
+    def _shaped(self, array, shape):
+        """``reshape`` within a call: no view (and no node of one) where there is
+        nothing to reshape."""
+        return array if isinstance(array, torch.Tensor) and array.shape == tuple(shape) else self.reshape(array, shape)
 
     def _as_input(self, x):
         if hasattr(x, "ndim") and hasattr(x, "shape"):
