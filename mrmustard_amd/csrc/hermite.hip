@@ -798,20 +798,28 @@ int launch_stable(const Shape &S, int64_t B, const double *A, const double *b, c
         return fail(MM_ERR_WORKSPACE, "stable workspace of %zu bytes needed, %zu given", stable_ws_bytes(S), ws_bytes);
     int nmax = 0;
     for (int j = 0; j < S.D; ++j) nmax += S.s[j] - 1;
-    // Per wavefront, one workgroup per triple loops over ceil(nrows / 1024)
-    // rows per thread, ~1.6 us per row and pivot axis beyond the first (one
-    // round per num_cu triples); a launch over all CUs costs ~5.5 us per triple
-    // and a microsecond per 130,000 terms ((20,)^5 12.7 us, (11,)^6 15 us).
+    // Per wavefront, one workgroup per triple (one round per num_cu triples)
+    // takes a microsecond per 1,100 terms of a triple, or what its passes over the
+    // rows cost; a launch over all CUs, one triple after another, a microsecond per
+    // 85,000 terms; both have a floor that grows with the dependent pivots.
+    // Measured: one workgroup (4,)^5 2.3 us a wavefront, (10,)^4 5.5, (16,)^4 19, (5,)^6
+    // 27, (25, 7, 3, 30, 2) 83; a launch (20,)^4 4.0, (40,)^4 5.5, (10,)^5 4.7, (20,)^5
+    // 12.7, (8,)^6 6.1, (11,)^6 15.
     const int64_t nrows = S.N / S.s[S.D - 1];
     const int64_t rounds = (B + ds->num_cu - 1) / ds->num_cu;
-    const double t_block = double((nrows + 1023) / 1024) * double(rounds) * 1.6 * std::max(1, S.D - 1);
     const double terms = double(S.N) * S.D * (S.D + 1) / std::max(1, nmax);
-    // The tiles (stable_tile.hpp) where their estimate is the least: all of
-    // D <= 5 that was tried, D = 6 up to about six per axis.
+    double t_block = double(rounds) * std::max({0.35 * (S.D + 1), 0.7 + terms / 1100.0, 1.3 * (S.D - 1) * double(nrows) / 1024.0});
+    double t_launch = double(B) * std::hypot(2.0 + 0.55 * S.D, terms / 85e3);
+    if (S.D > 6) {  // no tiles; a workgroup's step by its rows per thread
+        t_block = double(rounds) * double((nrows + 1023) / 1024) * 1.6 * (S.D - 1);
+        t_launch = 5.5 * double(B);
+    }
+    // The tiles (stable_tile.hpp) where their estimate is the least (the others
+    // and their row table cost 12 us besides).
     const Lat lat = lat_of(S);
     StableTilePlan tp;
     if (stable_tile_plan(lat, B, ws_bytes, ds, &tp) &&
-        (tp.whole() || S.D <= 2 || tp.us <= nmax * std::min(t_block, (5.5 + terms / 130e3) * double(B)))) {
+        (tp.whole() || S.D <= 2 || tp.us <= 12.0 + nmax * std::min(t_block, t_launch))) {
         int *nf = nullptr;
         if (!tp.whole()) {
             rc = nf_flag(s, &nf);
@@ -834,7 +842,7 @@ int launch_stable(const Shape &S, int64_t B, const double *A, const double *b, c
     a.tstride_a = int64_t(S.D) * S.D;
     a.tstride_b = S.D;
     a.tstride_g = S.N;
-    if (t_block <= 5.5 * double(B)) {
+    if (t_block <= t_launch) {
         a.A = reinterpret_cast<const double2 *>(A);
         a.b = reinterpret_cast<const double2 *>(b);
         a.c = reinterpret_cast<const double2 *>(c);

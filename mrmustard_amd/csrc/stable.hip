@@ -11,6 +11,10 @@ namespace {
 
 __global__ void clear_flag_kernel(int *nf) { *nf = 0; }
 
+// Blocks of a tile row in a launch of B triples: a multiple of the XCDs, so that
+// a triple stays on one.
+int64_t triple_lanes(int64_t B) { return (B + MM_XCDS - 1) / MM_XCDS * MM_XCDS; }
+
 // Fill p for tiles of at most e[j] points along axis j; false when the tile
 // does not fit one workgroup or the offsets their types.
 bool try_tiles(const Lat &g, int64_t B, size_t ws_bytes, const DevState *ds, const int (&e)[8], StableTilePlan *p) {
@@ -37,7 +41,7 @@ bool try_tiles(const Lat &g, int64_t B, size_t ws_bytes, const DevState *ds, con
             nrow *= p->e[j];
             trows *= n;
         }
-        if (cells > 16384 || nrow > STABLE_TILE_ROWS || trows * B > 0x7fffffff || reach > 0x7fffffff) return false;
+        if (cells > 16384 || nrow > STABLE_TILE_ROWS || trows * triple_lanes(B) > 0x7fffffff || reach > 0x7fffffff) return false;
     }
     const int64_t lanes = nrow * stable_lanes(D);
     p->cells = int(cells);
@@ -47,20 +51,45 @@ bool try_tiles(const Lat &g, int64_t B, size_t ws_bytes, const DevState *ds, con
     p->launches = int(launches);
     p->threads = int((lanes + MM_WAVE - 1) / MM_WAVE * MM_WAVE);
     p->shmem = size_t(cells) * 16 + size_t(p->e[L] + 1) * 16;
-    if (p->threads > 1024 || int64_t(p->shmem) > ds->max_lds || trows * B * p->threads > 0xffffffffll) return false;
+    if (p->threads > 1024 || int64_t(p->shmem) > ds->max_lds || trows * triple_lanes(B) * p->threads > 0xffffffffll) return false;
     if (p->whole()) return true;
     if (size_t(p->nhalo) * sizeof(StableHalo) > ws_bytes) return false;
     // A launch costs 3.5 us, a step 0.45 us and 0.01 us per wave, a halo cell
-    // 4 ns, a tile of a CU 1.2 us; tiles beyond those resident at once run in
-    // rounds (the middle launches have about 1.6 times the mean of tiles).
-    // Fitted to (40,)^4 in tiles of 3 to 6 points, (70, 70, 60), (1000, 1000),
-    // (20,)^5 and (11,)^6, which it meets to within 25 %.
+    // 4 ns: the time of one tile.  Tiles beyond about half of one per CU and
+    // launch (D = 6: any) share their CU; it gains from three of the smallest tiles
+    // and of those of D >= 5 at most, where they cost 1.3 to 1.7 times their share.  A
+    // block without a tile costs 0.2 ns a wave.  Meets (4,)^5 to (10,)^6, (20,)^3 to (20,)^4 and (40,)^4 in batches of 1 to
+    // 2,048 to within 25 %, a few to 40 %.
     const int waves = p->threads / MM_WAVE;
-    const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(ds->max_lds / int64_t(p->shmem), 16 / waves));
-    const double on_cu = tiles / double(launches) / ds->num_cu;
-    const double rounds = std::max(1.0, 1.6 * on_cu / double(per_cu));
-    p->us = double(launches) * (3.5 + 1.2 * on_cu + rounds * (0.004 * p->nhalo + double(steps) * (0.45 + 0.01 * waves)));
+    int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(ds->max_lds / int64_t(p->shmem), 16 / waves));
+    if (D >= 5 || (D == 4 && waves < 4)) per_cu = std::min<int64_t>(per_cu, 3);
+    const double tile = 0.004 * p->nhalo + double(steps) * (0.45 + 0.01 * waves);
+    const double shared = std::max(0.0, tiles / ds->num_cu - (D <= 5 ? 0.5 * double(launches) : 0.0));
+    const double idle = double(trows) * double(B) * double(launches) - tiles;
+    p->batch = B >= MM_XCDS && tiles > 0.4 * ds->num_cu * double(launches);
+    p->us = double(launches) * (3.5 + tile) + shared * tile / double(per_cu) * (D <= 4 ? 1.0 : (D == 5 ? 1.3 : 1.7)) + 0.2e-3 * waves * idle;
     return true;
+}
+
+template <int D, bool BATCH>
+int sweep_tiles(StableTileArgs &a, const StableTilePlan &p, int64_t B, void *ws, hipStream_t s) {
+    raise_lds_limit(stable_tile_kernel<D, BATCH>, int(p.shmem));
+    if (!a.whole) {
+        hipLaunchKernelGGL((stable_halo_kernel<D>), dim3(1), dim3(1024), 0, s, a, reinterpret_cast<StableHalo *>(ws));
+        LAUNCH_CHECK("stable_halo_kernel");
+    }
+    // BATCH from 0.4 tiles a CU and launch: (7,)^4 in batches of 64 66 -> 57 us, but (200, 200)
+    // in batches of 30 (0.27) 298 -> 310
+    for (a.w = 0; a.w < p.launches; ++a.w)
+        for (int64_t row = 0; row < (BATCH ? p.trows : 1); row += 65535) {  // grid y
+            a.row0 = int(row);
+            // launch w = 0 of one triple: its first tile row alone
+            const dim3 grid = BATCH ? dim3(unsigned(triple_lanes(B)), unsigned(std::min<int64_t>(65535, p.trows - row)))
+                                    : dim3(unsigned(a.w == 0 && B == 1 ? 1 : p.trows * B));
+            hipLaunchKernelGGL((stable_tile_kernel<D, BATCH>), grid, dim3(unsigned(p.threads)), p.shmem, s, a);
+            LAUNCH_CHECK("stable_tile_kernel");
+        }
+    return MM_OK;
 }
 
 }  // namespace
@@ -121,8 +150,9 @@ int launch_stable_tiles(const StableTilePlan &p, const Lat &g, int64_t B, const 
     a.cells = p.cells;
     a.nrow = p.nrow;
     a.trows = int(p.trows);
-    a.whole = p.whole();
+    a.ntriples = int(B);
     a.single = B == 1;
+    a.whole = p.whole();
     a.nhalo = p.nhalo;
     a.halo = reinterpret_cast<const StableHalo *>(ws);
     a.nf = nf;
@@ -130,28 +160,14 @@ int launch_stable_tiles(const StableTilePlan &p, const Lat &g, int64_t B, const 
         hipLaunchKernelGGL(clear_flag_kernel, dim3(1), dim3(1), 0, s, nf);
         LAUNCH_CHECK("clear_flag_kernel");
     }
-    for (int w = 0; w < p.launches; ++w) {
-        a.w = w;
-        // launch w = 0 of one triple: its first tile row alone
-        const unsigned grid = unsigned(w == 0 && B == 1 ? 1 : p.trows * B);
-        switch (g.D) {
-#define CASE(DD)                                                                                                             \
-    case DD:                                                                                                                 \
-        if (w == 0) {                                                                                                        \
-            raise_lds_limit(stable_tile_kernel<DD>, int(p.shmem));                                                           \
-            if (!a.whole)                                                                                                    \
-                hipLaunchKernelGGL((stable_halo_kernel<DD>), dim3(1), dim3(1024), 0, s, a, reinterpret_cast<StableHalo *>(ws)); \
-        }                                                                                                                    \
-        hipLaunchKernelGGL((stable_tile_kernel<DD>), dim3(grid), dim3(unsigned(p.threads)), p.shmem, s, a);                  \
-        break;
-            CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6)
+    switch (g.D) {
+#define CASE(DD) \
+    case DD: return p.batch ? sweep_tiles<DD, true>(a, p, B, ws, s) : sweep_tiles<DD, false>(a, p, B, ws, s);
+        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6)
 #undef CASE
-            default:
-                return fail(MM_ERR_INVALID, "bad D");
-        }
-        LAUNCH_CHECK("stable_tile_kernel");
+        default:
+            return fail(MM_ERR_INVALID, "bad D");
     }
-    return MM_OK;
 }
 
 }  // namespace mm

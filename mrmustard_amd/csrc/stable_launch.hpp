@@ -12,6 +12,7 @@ struct StableTilePlan {
     int64_t trows = 0;
     size_t shmem = 0;
     double us = 0.0;  // estimated time
+    bool batch = false;
     bool whole() const { return launches == 1; }
 };
 
