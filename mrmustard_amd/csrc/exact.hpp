@@ -132,20 +132,24 @@ __device__ void exact_forward(const Ops &t, const Lat &g, int top, const double2
 // reach any earlier flat position, so no two points are independent a priori.
 // A negative index wraps around the lattice; it reads a value only when that
 // position is already written (earlier in flat order), else zero, as the
-// reference's zero-initialised G holds there.
-template <class Ops>
+// reference's zero-initialised G holds there.  DD = g.D: unrolled over the axes,
+// one (7,)^4 in 4.4 ms against 9.2.
+template <int DD, class Ops>
 __device__ void exact_stable_forward(const Ops &t, const Lat &g, const double2 *A, const double2 *b, double2 c, double2 *G,
                                      const double *sq) {
     if (t.rank == 0) {
-        const int D = g.D;
+        constexpr int D = DD;
         const int64_t N = g.N;
         const double2 zero = make_double2(0.0, 0.0);
-        int k[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        int k[D] = {};
         G[0] = c;
         for (int64_t p = 1; p < N; ++p) {
-            for (int a = D - 1; a >= 0; --a) {  // np.ndindex order
-                if (++k[a] < g.shape[a]) break;
-                k[a] = 0;
+            bool up = true;  // np.ndindex order
+#pragma unroll
+            for (int a = D - 1; a >= 0; --a) {
+                k[a] += up;
+                up = up && k[a] == g.shape[a];
+                if (up) k[a] = 0;
             }
             auto rd = [&](int64_t q) {
                 if (q < 0) q += N;
@@ -153,13 +157,16 @@ __device__ void exact_stable_forward(const Ops &t, const Lat &g, const double2 *
             };
             int num = 0;
             double2 vals = zero;
+#pragma unroll
             for (int i = 0; i < D; ++i) {
                 if (k[i] == 0) continue;
                 ++num;
                 const int64_t pivot = p - g.stride[i];
                 double2 val = cmul(b[i], G[pivot]);
+#pragma unroll
                 for (int j = 0; j < i; ++j) val = cadd(val, cmul(cscale_promoted(A[i * D + j], sq[k[j]]), rd(pivot - g.stride[j])));
                 val = cadd(val, cmul(cscale_promoted(A[i * D + i], sq[k[i] - 1]), rd(pivot - g.stride[i])));
+#pragma unroll
                 for (int j = i + 1; j < D; ++j) val = cadd(val, cmul(cscale_promoted(A[i * D + j], sq[k[j]]), rd(pivot - g.stride[j])));
                 vals = cadd(vals, cdiv_promoted(val, sq[k[i]]));
             }

@@ -300,7 +300,7 @@ __global__ __launch_bounds__(1024) void stable_tile_kernel(StableTileArgs a) {
     const bool any = __syncthreads_or(bad);
     if (a.whole) {
         // non-finite values: the reference's sequential sweep with every term
-        if (any) exact_stable_forward(BlockOps(red), a.g, A, b, c, G, a.sq);
+        if (any) exact_stable_forward<D>(BlockOps(red), a.g, A, b, c, G, a.sq);
     } else if (threadIdx.x == 0) {
         if (a.single && a.w == 0) *a.nf = any;
         else if (any) atomicOr(a.nf, 1);
