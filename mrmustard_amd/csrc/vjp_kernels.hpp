@@ -174,7 +174,7 @@ __device__ __forceinline__ void vjp_group(const VjpArgs &a, const double *sqt, i
     // I32: the points' byte offsets from the arrays' (uniform) addresses fit 32
     // bits.  Half of the kernel's issue slots were busy, a third of them with 64-bit
     // addresses: a slab of 10^7 points of D = 8 with the next one formed 367 -> 322 us
-    // (1.1 GB, 3.5 TB/s), (12,)^6 52.5 -> 48.
+    // (1.9 GB read, 0.16 written: 6.4 TB/s), (12,)^6 52.5 -> 48.
     using X = std::conditional_t<I32, uint32_t, int64_t>;
     auto at = [](const double2 *p, X x) {
         if constexpr (I32) return *reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(p) + x * 16u);
@@ -287,8 +287,12 @@ __device__ __forceinline__ void vjp_group(const VjpArgs &a, const double *sqt, i
     block_store_group<D, R0, R1>(held, row, SLAB && m > 0);
 }
 
+// Waves per SIMD held to what the loads of a whole point need: left to aim
+// higher, the compiler moves them to their uses ((20,)^5 41 -> 73 us, 96 of (12,)^4 27 ->
+// 36; held, 39 and 25.5).
 template <int D, bool SLAB, bool FWD, bool LT, bool I32>
-__global__ __launch_bounds__(256, D <= 4 ? 3 : 2) void vjp_kernel(VjpArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 4 ? 3 : 2, D <= 2 ? 8 : (D == 3 ? 4 : (D == 4 ? 3 : 2))))) void
+vjp_kernel(VjpArgs a) {
     extern __shared__ double sqt[];
     using RS = RowSplit<D>;
     if (LT) {
