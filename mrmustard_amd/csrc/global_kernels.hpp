@@ -372,11 +372,6 @@ __global__ __launch_bounds__(256) void fwd_slab0_kernel(Slab0Args a) {
     }
 }
 
-__global__ void zero_c128_kernel(double2 *p, int64_t n) {
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
-        p[i] = make_double2(0.0, 0.0);
-}
-
 // ------------------------------------------------------------- stable sweep
 // core.py:183-211.  All pivots of a point lie on the previous index-sum
 // wavefront, so the lattice is swept by |k| = n.  A "row" fixes k_0..k_{D-2};

@@ -639,19 +639,22 @@ size_t vjp_rows_bytes(const Shape &S, int64_t B, int chunks) { return size_t(B) 
 
 size_t vjp_min_ws_bytes(const Shape &S, int64_t B) { return vjp_rows_bytes(S, B, vjp_chunks_min_ws(S.N, B)); }
 
+// CUs that a VJP's workspace is sized for (the whole chip).
+constexpr int VJP_CUS = 256;
+
 // Blocks per triple and row group over `points` points: at least two points
-// per thread, and no more blocks than are resident at a time (D <= 4: four
-// per CU, D <= 6: two, D >= 7: one per row group), so that all of them advance
-// through the lattice together; a multiple of the XCD count.
-int vjp_chunks(int D, int64_t points, int64_t B) {
-    const int64_t cap = std::max<int64_t>(1, (D <= 4 ? 1024 : (D <= 6 ? 512 : 256)) / std::max<int64_t>(B, 1));
+// per thread, and about as many blocks as are resident at a time (D <= 4: four
+// per CU, of which D = 4 holds three; D <= 6: two, D >= 7: one per row group), so that
+// they advance through the lattice together; a multiple of the XCD count.
+int vjp_chunks(int D, int64_t points, int64_t B, int num_cu) {
+    const int64_t cap = std::max<int64_t>(1, (D <= 4 ? 4 : (D <= 6 ? 2 : 1)) * std::min(num_cu, VJP_CUS) / std::max<int64_t>(B, 1));
     int64_t n = std::max<int64_t>(1, std::min<int64_t>((points + 511) / 512, cap));
     if (n > MM_XCDS) n -= n % MM_XCDS;
     return int(n);
 }
 
 size_t vjp_ws_bytes(const Shape &S, int64_t B) {
-    return std::max(vjp_min_ws_bytes(S, B), vjp_rows_bytes(S, B, vjp_chunks(S.D, S.N, B)));
+    return std::max(vjp_min_ws_bytes(S, B), vjp_rows_bytes(S, B, vjp_chunks(S.D, S.N, B, VJP_CUS)));
 }
 
 template <int D, bool SLAB, bool FWD>
@@ -690,7 +693,7 @@ int launch_vjp_sums(const Shape &S, int64_t B, const double *G, const double *g,
                     void *ws, size_t ws_bytes, bool conj, const DevState *ds, hipStream_t s) {
     if (!ws || ws_bytes < vjp_min_ws_bytes(S, B))
         return fail(MM_ERR_WORKSPACE, "VJP workspace of %zu bytes needed, %zu given", vjp_ws_bytes(S, B), ws_bytes);
-    int nchunk = vjp_chunks(S.D, S.N, B);
+    int nchunk = vjp_chunks(S.D, S.N, B, ds->num_cu);
     if (ws_bytes < vjp_rows_bytes(S, B, nchunk)) nchunk = std::min(nchunk, vjp_chunks_min_ws(S.N, B));
     VjpArgs a = vjp_args(S, ws, nchunk, S.N, conj, ds);
     a.G = reinterpret_cast<const double2 *>(G);
@@ -893,7 +896,7 @@ int launch_stable(const Shape &S, int64_t B, const double *A, const double *b, c
 
 // Workspace of one vanilla forward (+ fused VJP when `fused`).
 // A single triple (D >= 3) whose level-0 slab fits in LDS but holds more
-// points than FACE_POINTS (with the VJP, more than 1024) is swept over all CUs:
+// points than face_points() (with the VJP, more than 1024) is swept over all CUs:
 // the face {k_0 = 0} in LDS (team size *Tf), then the level-0 slabs.  Measured
 // for the forward: (100, 50, 50) 189 -> 113 us, (40,)^3 70 -> 64 us, but
 // (30, 35, 40) 48 -> 51 us; a fused workgroup step adds the VJP terms.
@@ -992,7 +995,7 @@ int vanilla_uniform(const Shape &S, int64_t B, const double *A, const double *b,
         }
         if (fuse_level0) {
             double2 *G2 = sa.G;
-            const int nchunk = std::min(vjp_chunks(S.D, S.st[0], 1), vjp_chunks_min_ws(S.N, 1));
+            const int nchunk = std::min(vjp_chunks(S.D, S.st[0], 1, ds->num_cu), vjp_chunks_min_ws(S.N, 1));
             rc = launch_level0_vjp(S, A + 2 * t * a.ua, b + 2 * t * a.ub, c + 2 * t, g + 2 * t * a.ug,
                                    [G2, &S](int m) { return G2 + int64_t(m) * S.st[0]; }, dA + 2 * t * a.ua, db + 2 * t * a.ub, dc + 2 * t,
                                    ws, nchunk, ds, s);
@@ -1011,10 +1014,10 @@ int vanilla_uniform(const Shape &S, int64_t B, const double *A, const double *b,
 // ------------------------------------------------------- recompute VJP path
 //
 // dL/dA, dL/db, dL/dc from (A, b, c, dL/dG) without the whole of G in
-// memory: the face k_0 = 0 is computed into window slot 0, then each level-0
-// slab m is recomputed into slot m % 3 from slots (m-1) % 3 and (m-2) % 3 and
-// its VJP terms are added to per-block partial sums.  Resident memory is
-// three slabs (3 * stride[0] * 16 B) instead of the lattice.  Lattices of at
+// memory: the face k_0 = 0 is computed into window slot 0, then one launch per
+// level-0 slab m reads slots m % 3 and (m-1) % 3 and the cotangent's slabs m and
+// m + 1, adds the VJP terms of slab m to per-block partial sums and writes slab
+// m + 1 to slot (m+1) % 3.  Resident memory is three slabs (3 * stride[0] * 16 B) instead of the lattice.  Lattices of at
 // most 64 MB, and those whose slabs fit in LDS, take the fused sweep with a
 // full G in the workspace (recompute_whole).
 
@@ -1130,7 +1133,7 @@ int vjp_recompute(const Shape &S, const double *A, const double *b, const double
     if (rc) return rc;
     // 2. level 0: the VJP terms of slab m with slab m + 1, then the sums' end
     return launch_level0_vjp(S, A, b, c, g, [&slot](int m) { return slot[m % 3]; }, dA, db, dc, partial,
-                             std::min(vjp_chunks(S.D, S.st[0], 1), recompute_rows(S, ds)), ds, s);
+                             std::min(vjp_chunks(S.D, S.st[0], 1, ds->num_cu), recompute_rows(S, ds)), ds, s);
 }
 
 // ------------------------------------------------------------------- plans

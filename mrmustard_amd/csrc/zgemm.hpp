@@ -36,7 +36,7 @@ struct ZgemmArgs {
 
 constexpr int ZG_BN = 128, ZG_BK = 8;
 
-// Two workgroups per CU.  Large products only (strip_plan): measured 64.5
+// Two workgroups per CU.  Large products only (strip_rt): measured 64.5
 // TFLOP/s at 2048^3 and 65.4 at 4096^3, where zgemm_strip_kernel has 61.3 and 64.3.
 __global__ __launch_bounds__(256, 2) void zgemm_mfma_kernel(ZgemmArgs a) {
     constexpr int ZG_BM = 64;
