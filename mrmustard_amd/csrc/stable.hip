@@ -11,9 +11,9 @@ namespace {
 
 __global__ void clear_flag_kernel(int *nf) { *nf = 0; }
 
-// Blocks of a tile row in a launch of B triples: a multiple of the XCDs, so that
-// a triple stays on one.
-int64_t triple_lanes(int64_t B) { return (B + MM_XCDS - 1) / MM_XCDS * MM_XCDS; }
+// Blocks of a tile row in a launch of B triples: from one per XCD a multiple of the
+// XCDs, so that a triple stays on one.
+int64_t triple_lanes(int64_t B) { return B < MM_XCDS ? B : (B + MM_XCDS - 1) / MM_XCDS * MM_XCDS; }
 
 // Fill p for tiles of at most e[j] points along axis j; false when the tile
 // does not fit one workgroup or the offsets their types.
